@@ -5,8 +5,9 @@
 // tiles past the last visible key are never touched, the online softmax runs in
 // base 2 with c = scale*log2(e), and a row that sees no key is exactly 0.
 //
-// bf16 (flash_bf16_p64_kernel, the default): 4 waves x 64 query rows per block,
-// one wave per SIMD.  A wave's VALU work runs while its own independent MFMAs
+// bf16 calls take one of two tiled kernels (duo_plan in ca_duo.h): flash_duo_kernel
+// for most, and for long E = 128 walks that fill the chip flash_bf16_p64_kernel: 4
+// waves x 64 query rows per block, one wave per SIMD.  A wave's VALU work runs while its own independent MFMAs
 // execute, so each wave issues one stream per key tile of 64: the P.V MFMAs of
 // the previous tile, the S MFMAs of the next and the softmax of this one.  Key
 // tiles go global -> LDS with direct buffer loads; K is read with ds_read_b128,
@@ -1348,18 +1349,24 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p) {
   }  // passes
 }
 
-template <typename K>
+template <typename K, typename... A>
 static int launch_lds(K kernel, int64_t nb, int threads, int lds, const FlashParams& p, hipStream_t stream,
-                      int64_t ny = 1) {
+                      int64_t ny = 1, A... args) {
   if (nb > 0x7fffffff || ny > 0xffff) return CA_DECLINED;
   if (lds > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return CA_HIP_ERROR - (int)e;
   }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)nb, (unsigned)ny), dim3(threads), lds, stream, p);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)nb, (unsigned)ny), dim3(threads), lds, stream, p, args...);
   return ca_launch_status();
 }
+
+}  // namespace ca
+
+#include "ca_duo.h"
+
+namespace ca {
 
 FlashPlan flash_plan(const FlashParams& p, int E, bool bf16) {
   FlashPlan plan{};
@@ -1397,6 +1404,24 @@ FlashPlan flash_plan(const FlashParams& p, int E, bool bf16) {
   return plan;
 }
 
+// A tiled bf16 call: the duo kernel or the 64-row kernel (duo_plan), then the combine
+// of a split call's partials.  Either's splits number at most plan.splits, whose
+// partials the workspace holds.
+template <int E>
+static int bf16_launch(const FlashParams& p, const FlashPlan& plan, hipStream_t stream) {
+  const DuoPlan d = duo_plan(p, E, plan);
+  const int64_t splits = d.kg ? d.splits : plan.splits;
+  constexpr int threads = 64 * FlashP64Cfg<E>::NW, lds = FlashP64Cfg<E>::LDS_BYTES;
+  int st;
+  if (d.kg)
+    st = duo_launch<E>(p, d, stream);
+  else if (plan.split)
+    st = launch_lds(flash_bf16_p64_kernel<E, true>, plan.gx, threads, lds, p, stream, splits);
+  else
+    st = launch_lds(flash_bf16_p64_kernel<E, false>, plan.gx, threads, lds, p, stream);
+  return st == CA_OK && splits > 1 ? flash_combine_launch(p, E, true, splits, stream) : st;
+}
+
 int flash_launch(const FlashParams& p, int E, int bf16, hipStream_t stream) {
   const FlashPlan plan = flash_plan(p, E, bf16 != 0);
   if (plan.kind == kPlanNone) return CA_OK;
@@ -1407,20 +1432,10 @@ int flash_launch(const FlashParams& p, int E, int bf16, hipStream_t stream) {
   if (plan.kind == kPlanSmall) return flash_small_launch(p, plan, E, stream);
   const int64_t nb = plan.gx, splits = plan.splits;
   if (bf16) {
-    if (plan.split) {
-      int st = CA_DECLINED;
-      switch (E) {
-        case 32: st = launch_lds(flash_bf16_p64_kernel<32, true>, nb, 64 * FlashP64Cfg<32>::NW, FlashP64Cfg<32>::LDS_BYTES, p, stream, splits); break;
-        case 64: st = launch_lds(flash_bf16_p64_kernel<64, true>, nb, 64 * FlashP64Cfg<64>::NW, FlashP64Cfg<64>::LDS_BYTES, p, stream, splits); break;
-        case 128: st = launch_lds(flash_bf16_p64_kernel<128, true>, nb, 64 * FlashP64Cfg<128>::NW, FlashP64Cfg<128>::LDS_BYTES, p, stream, splits); break;
-      }
-      if (st != CA_OK) return st;
-      return flash_combine_launch(p, E, bf16, splits, stream);
-    }
     switch (E) {
-      case 32: return launch_lds(flash_bf16_p64_kernel<32, false>, nb, 64 * FlashP64Cfg<32>::NW, FlashP64Cfg<32>::LDS_BYTES, p, stream);
-      case 64: return launch_lds(flash_bf16_p64_kernel<64, false>, nb, 64 * FlashP64Cfg<64>::NW, FlashP64Cfg<64>::LDS_BYTES, p, stream);
-      case 128: return launch_lds(flash_bf16_p64_kernel<128, false>, nb, 64 * FlashP64Cfg<128>::NW, FlashP64Cfg<128>::LDS_BYTES, p, stream);
+      case 32: return bf16_launch<32>(p, plan, stream);
+      case 64: return bf16_launch<64>(p, plan, stream);
+      case 128: return bf16_launch<128>(p, plan, stream);
     }
   } else {
     if (plan.split) {

@@ -131,6 +131,10 @@ constexpr int kRowsWaves = 8;                 // waves per block
 constexpr int64_t kRowsTargetBlocks = 256;    // blocks that keep every CU streaming
 constexpr int64_t kRowsMaxSplits = 64;
 
+// The bf16 rule below is flash_bf16_p64_kernel's, and sets the workspace of every bf16
+// call; duo_plan (ca_duo.h) decides which calls run that kernel and how many splits,
+// at most these, the others use.
+//
 // The tiled prefill splits each query block's keys over several blocks when its
 // query blocks (batch x heads x ceil(seq_q / rows per block): 256 rows in bf16,
 // 128 in fp32) leave the chip's CUs short of blocks: about kTiledTargetBlocks

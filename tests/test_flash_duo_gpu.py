@@ -1,0 +1,44 @@
+"""flash_duo_kernel on the GPU at the edges of its tiles and of duo_plan's rules, with
+and without rows that take the safe walk, against the float64 oracle on sampled rows."""
+
+import random
+
+import numpy as np
+import pytest
+import torch
+
+from cpu_attention import flash_attn_func
+from helpers import assert_close, values
+from oracle.attention import attention
+from test_duo_geometry import EDGES
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("gap", [0, 180])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("shape", EDGES)
+def test_edges(cuda, shape, d, causal, gap):
+    """gap: a key past the first tiles whose logits exceed theirs by about that many
+    log2 units in every other head, past the fixed max's headroom, so that some blocks
+    walk twice (both key groups, both passes of a pair, every split)."""
+    b, sq, sk, h = shape
+    print(f"duo edges {shape} d={d} causal={causal} gap={gap}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(sq + sk + d)
+    q, k, v = (torch.randn(b, h, n, d, generator=g, device=cuda).transpose(1, 2) for n in (sq, sk, sk))
+    if gap:
+        q = q + 1.0
+        k[:, sk * 2 // 3, ::2] = (gap + 4) / (1.4427 * d ** 0.5)
+    q, k, v = (x.bfloat16() for x in (q, k, v))
+    out = flash_attn_func(q, k, v, causal=causal)
+    r = random.Random(sq * sk + d)
+    rows = sorted({0, sq - 1, min(sq - 1, 127), *(r.randrange(sq) for _ in range(12))})
+    pairs = {(0, 0), (b - 1, h - 1), *((r.randrange(b), r.randrange(h)) for _ in range(3))}
+    for bi, hi in sorted(pairs):
+        qv, kv, vv, ov = (values(t[bi:bi + 1, :, hi:hi + 1]) for t in (q, k, v, out))
+        ref = []
+        for i in rows:
+            ke = min(sk, max(0, i + 1 + sk - sq)) if causal else sk
+            ref.append(attention(qv[:, i:i + 1], kv[:, :ke], vv[:, :ke], d ** -0.5)[0, 0, 0] if ke else np.zeros(d))
+        assert_close(torch.from_numpy(ov[0, rows, 0]), np.stack(ref), torch.bfloat16, paged=False)
