@@ -1,0 +1,381 @@
+// fp32 prefill on the fp16 matrix instructions (included by ca_flash.hip).
+//
+// The 32-bit MFMA (32x32x2: 64 cycles per 4 KFLOP) bounds fp32 attention at 157 TFLOP/s
+// and sums 128 terms of a logit one pair at a time.  Here every fp32 operand x is split
+// into two fp16 values, high = fp16(x) and low = fp16(x - high), which hold 23 of its 24
+// significant bits (24 where the low one needs at most 11), and a product takes three
+// 32x32x16 fp16 MFMAs with fp32 sums: high.high + high.low + low.high (the low.low term
+// is below 2^-24 of the product).  That is 96 instead of 512 cycles.  Probabilities,
+// their sums and the output stay fp32; P is split in the same way for P.V.
+//
+// Precision.  Against 64 bits the split kernel is closer than the 32-bit MFMAs, whose
+// long chains of sums cost more than the splits (2-norm errors, N(0, 1) inputs, before
+// -> now): N=1 L=S=2048 H=32 E=128 causal 4.6e-7 -> 3.1e-7, L=S=4096 non-causal 1.2e-6
+// -> 7.8e-7, L=S=1024 H=16 E=64 causal 2.9e-7 -> 2.3e-7; with q 8 times larger (peaked
+// rows, E=64) 8.8e-7 -> 5.5e-7; with lognormal, shifted or per-channel scaled K and V it
+// is lower too.  Over few keys the chains are short and the splits would lose up to 45 %
+// (E=64 L=S=17 causal 1.2e-7 -> 1.7e-7): f32_exact leaves those calls to the 32-bit MFMAs.
+//
+// Range.  fp16 reaches from 2^-24 to 65504, so the operands are scaled by powers of two:
+// each Q row by its own maximum, K and V by that of the block's first tile, to [2^10,
+// 2^11); p by 2^10 (2^14 between two refreshes of the running max).  A block whose
+// values leave that range (a later tile's maximum 2^5 above or 2^14 below the first's, a
+// magnitude outside 2^+-40, inf or NaN) redoes the query block with the 32-bit MFMAs
+// (f32_safe_pass), so such inputs give what they gave before.
+//
+// Bound: the three MFMAs per product and the splitting of K and V tiles by every block
+// of 128 rows.  Measured back to back, before -> now: N=1 L=S=2048 H=32 E=128 causal 330
+// -> 171 us (201 TFLOP/s), N=1 L=S=4096 non-causal 2094 -> 947 us (290 TFLOP/s), N=4
+// L=S=4096 H=32 E=64 causal 2266 -> 1136 us, N=8 L=S=512 H=16 E=64 81 -> 43 us, N=1 L=64
+// S=4096 H=8 E=64 30 -> 21 us.
+#pragma once
+
+namespace ca {
+
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4v;
+typedef __attribute__((address_space(3))) s16x4v lds_s16x4;
+
+template <int E>
+struct F32Cfg {
+  static constexpr int BN = 32;           // keys per tile
+  static constexpr int PL = BN * E * 2;   // bytes of one plane (high or low halves) of a tile
+  static constexpr int TB = 4 * PL;       // K high, K low, V high, V low
+  static constexpr int CH = FlashF32Cfg<E>::CH;
+  static constexpr int LDS_BYTES = 2 * TB > FlashF32Cfg<E>::LDS_BYTES ? 2 * TB : FlashF32Cfg<E>::LDS_BYTES;
+};
+
+__device__ __forceinline__ uint32_t f16_bits(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
+// a and b, each as two fp16 values high + low (rounded to nearest even).
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  const f16x2 h = {static_cast<_Float16>(a), static_cast<_Float16>(b)};
+  hi = f16_bits(h);
+  lo = f16_bits(f16x2{static_cast<_Float16>(a - static_cast<float>(h.x)), static_cast<_Float16>(b - static_cast<float>(h.y))});
+}
+
+// The larger magnitude of each half of two fp16 pairs (as bits: inf and NaN are largest).
+__device__ __forceinline__ uint32_t max_abs16(uint32_t top, uint32_t x) {
+  typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, top),
+                                                                __builtin_bit_cast(u16x2, x & 0x7fff7fffu)));
+}
+
+// The exponent of a finite nonzero |x| = 2^e * [1, 2), as bits; 0 for 0.
+__device__ __forceinline__ int exp_of(float mx) { return (int)((__float_as_uint(mx) >> 23) & 255) - 127; }
+
+constexpr int kF32Top = 10;  // the scaled block maximum lies in [2^10, 2^11)
+
+// The power of two that scales values up to mx to kF32Top, and whether the values are
+// ones the split holds: not past 2^40 (nor inf or NaN), nor, unless all are 0, below 2^-40.
+__device__ __forceinline__ float f32_scale(float mx, bool& ok) {
+  const int e = exp_of(mx);
+  ok = mx == 0.f || (e >= -40 && e <= 40);
+  return mx == 0.f || !ok ? 1.f : __uint_as_float((uint32_t)(127 + kF32Top - e) << 23);
+}
+
+// Calls of few keys stay on the 32-bit MFMAs, which are closer to 64 bits there and no
+// slower (E=32 L=S=17: 4.3 against 5.4 us; E=32 L=S=200 causal error 1.9e-7 against
+// 2.0e-7, non-causal from 48 keys
+// lower; E=64 L=S=32 causal 1.57e-7 against 1.68e-7, from 40 keys even).
+inline bool f32_exact(int E, bool causal, int64_t seq_k) {
+  return E == 32 ? seq_k <= (causal ? 192 : 32) : E == 64 && seq_k <= 32;
+}
+
+template <int E, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pair) {
+  using C = F32Cfg<E>;
+  constexpr int BN = C::BN, PL = C::PL, TB = C::TB, CH = C::CH, NS = E / 16, ND = E / 32;
+  extern __shared__ __attribute__((aligned(1024))) char f32_smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int li = lane & 31, hf = lane >> 5;
+  PairWork pw{};
+  if (pair) pw = pair_work(p, kBM, false, blockIdx.x);
+  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((const lds_void*)f32_smem);
+  const int sp = SPLIT ? (int)blockIdx.y : 0, splits = SPLIT ? (int)gridDim.y : 1;
+  // LDS address of this thread's first staged chunk (8 bytes of halfs): K and V rows,
+  // swizzled as the bf16 tiles; chunk i lies RI rows further (at E = 128 every other
+  // one with another K swizzle).
+  constexpr int RI = 1024 / E;
+  const int cr = tid / (E / 4), c4 = tid % (E / 4), col = c4 >> 1;
+  const uint32_t kst = lds0 + cr * 2 * E + ((col ^ duo_k_swz<E>(cr)) << 4) + (c4 & 1) * 8;
+  const uint32_t vst = lds0 + 2 * PL + cr * 2 * E + ((((col >> 2) ^ duo_v_swz<E>(cr)) << 2 | (col & 3)) << 4) + (c4 & 1) * 8;
+  const uint32_t kl = lds0 + li * 2 * E + ((hf ^ duo_k_swz<E>(li)) << 4);
+  const int j = lane & 15, dh = (lane >> 4) & 1;
+  uint32_t va[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+    va[d] = lds0 + 2 * PL + (4 * hf + (j >> 2)) * 2 * E + ((d ^ duo_v_swz<E>(j >> 2)) << 6) + dh * 32 + (j & 3) * 8;
+
+  const int np = pair ? pw.n : 1;
+  uint32_t failed = 0;  // passes whose values the split operands do not hold
+#pragma unroll 1
+  for (int pass = 0; pass < np; ++pass) {
+    if (pass > 0) __syncthreads();  // the tile buffers of the pass before are free
+    const BlockWork bw = pair ? BlockWork{pw.b, pw.h, (pass ? pw.qb1 : pw.qb0) * kBM} : block_work(p, blockIdx.x);
+    const int L = (int)p.seq_q, S = (int)p.seq_k, diag = S - L;
+    const float* qg = reinterpret_cast<const float*>(p.q) + bw.b * p.qs[0] + bw.h * p.qs[2];
+    const float* kg = reinterpret_cast<const float*>(p.k) + bw.b * p.ks[0] + bw.h * p.ks[2];
+    const float* vg = reinterpret_cast<const float*>(p.v) + bw.b * p.vs[0] + bw.h * p.vs[2];
+    const int r0 = (int)bw.q0 + 32 * wv, row = r0 + li;
+    const F32Keys kr = f32_keys(p, bw.q0, SPLIT, sp, splits);
+    const int nkt = kr.nkt, kbeg = (int)kr.kbeg;
+    const int kend_w = p.causal ? imin(S, r0 + 32 + diag) : S;
+
+    // Tiles: global -> registers (buffer loads rebased at each tile, zeros past the
+    // last key), split into LDS planes by store_one.
+    u32x4 reg[CH];
+    const int koff = f32_tile_offset<E>(tid, 0, p.ks[1]), voff = f32_tile_offset<E>(tid, 0, p.vs[1]);
+    const int kstep = (int)(RI * p.ks[1] * 4), vstep = (int)(RI * p.vs[1] * 4);
+    auto load_one = [&](const float* g, int64_t stride, int off, int step, int t, u32x4 (&x)[CH]) __attribute__((always_inline)) {
+      const int64_t k0 = kbeg + (int64_t)t * BN;
+      const __amdgpu_buffer_rsrc_t rs = tile_rsrc(g + k0 * stride, f32_tile_bytes<E>(S, k0, stride));
+      asm volatile("" : "+v"(off));  // the chunks' offsets are added here, not kept
+#pragma unroll
+      for (int i = 0; i < CH; ++i) x[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + i * step, 0, 0);
+    };
+    auto load_k = [&](int t, u32x4 (&x)[CH]) __attribute__((always_inline)) { load_one(kg, p.ks[1], koff, kstep, t, x); };
+    auto load_v = [&](int t, u32x4 (&x)[CH]) __attribute__((always_inline)) { load_one(vg, p.vs[1], voff, vstep, t, x); };
+    bool ok = true;  // every value so far is one the split operands hold
+    float sk = 1.f, sv = 1.f;
+    // Splits this thread's staged values into the planes of a tile buffer.
+    auto store_one = [&](const u32x4 (&x)[CH], float sc, uint32_t at0, bool k) __attribute__((always_inline)) {
+      uint32_t top = 0;
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        u32x2 hi, lo;
+        uint32_t h, l;
+        split2(__uint_as_float(x[i].x) * sc, __uint_as_float(x[i].y) * sc, h, l);
+        hi.x = h;
+        lo.x = l;
+        split2(__uint_as_float(x[i].z) * sc, __uint_as_float(x[i].w) * sc, h, l);
+        hi.y = h;
+        lo.y = l;
+        const uint32_t at = (k && E == 128 && (i & 1) ? at0 ^ 128u : at0) + i * RI * 2 * E;
+        *(lds_u32x2*)(uintptr_t)at = hi;
+        *(lds_u32x2*)(uintptr_t)(at + PL) = lo;
+        top = max_abs16(max_abs16(top, hi.x), hi.y);
+      }
+      const uint32_t big = (top & 0xffff) > (top >> 16) ? top & 0xffff : top >> 16;
+      // fp16 0x2c00 = 2^-4: the wave's values reach within 2^-15 of the block's maximum.
+      ok &= !__any(big >= 0x7c00u) && (__any(big >= 0x2c00u) || !__any(big != 0u));
+    };
+    auto store_k = [&](const u32x4 (&x)[CH], int buf) __attribute__((always_inline)) { store_one(x, sk, kst + buf * TB, true); };
+    auto store_v = [&](const u32x4 (&x)[CH], int buf) __attribute__((always_inline)) { store_one(x, sv, vst + buf * TB, false); };
+
+    u32x4 vreg0[CH];
+    if (nkt > 0) {
+      load_k(0, reg);
+      load_v(0, vreg0);
+    }
+    // Q, scaled per row: lane (row li, half hf) holds dims 16 s + 8 hf .. +7.
+    f16x8 qh[NS], ql[NS];
+    float c = 0.f;
+    {
+      float qv[NS][8];
+      uint32_t mb = 0;  // the row's largest magnitude, as bits (inf and NaN are largest)
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          u32x4 v = {0, 0, 0, 0};
+          if (row < L) v = *reinterpret_cast<const u32x4*>(qg + (int64_t)row * p.qs[1] + 16 * s + 8 * hf + 4 * u);
+          const float f[4] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            qv[s][4 * u + x] = f[x];
+            mb = umax(mb, __float_as_uint(f[x]) & 0x7fffffffu);
+          }
+        }
+      const float mx = __uint_as_float(umax(mb, __shfl_xor(mb, 32)));
+      bool fits;
+      // A negative softmax scale turns Q's sign instead, and a zero one zeroes Q, so
+      // that c > 0: the running max is taken of the raw logits, and -inf * c is -inf.
+      float sq = f32_scale(mx, fits);
+      ok &= __all(fits);
+      c = fabsf(p.c) / sq;
+      sq = p.c < 0.f ? -sq : sq;
+      if (p.c == 0.f) {
+        sq = 0.f;
+        c = 1.f;
+      }
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        u32x4 h, l;
+        uint32_t a, b;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          split2(qv[s][2 * x] * sq, qv[s][2 * x + 1] * sq, a, b);
+          h[x] = a;
+          l[x] = b;
+        }
+        qh[s] = __builtin_bit_cast(f16x8, h);
+        ql[s] = __builtin_bit_cast(f16x8, l);
+      }
+    }
+    // The block's K and V scales, from its first tile.
+    if (nkt > 0) {
+      uint32_t mk = 0, mv = 0;
+#pragma unroll
+      for (int i = 0; i < CH; ++i)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const uint32_t a = reg[i][x] & 0x7fffffffu, b = vreg0[i][x] & 0x7fffffffu;
+          mk = umax(mk, a);
+          mv = umax(mv, b);
+        }
+#pragma unroll
+      for (int x = 32; x > 0; x >>= 1) {
+        const uint32_t a = __shfl_xor(mk, x), b = __shfl_xor(mv, x);
+        mk = umax(mk, a);
+        mv = umax(mv, b);
+      }
+      uint32_t* w = reinterpret_cast<uint32_t*>(f32_smem);
+      if (lane == 0) {
+        w[2 * wv] = mk;
+        w[2 * wv + 1] = mv;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        mk = umax(mk, w[2 * x]);
+        mv = umax(mv, w[2 * x + 1]);
+      }
+      __syncthreads();
+      bool fk, fv;
+      sk = f32_scale(__uint_as_float(mk), fk);
+      sv = f32_scale(__uint_as_float(mv), fv);
+      ok &= fk && fv;
+      c /= sk;
+      store_k(reg, 0);
+      store_v(vreg0, 0);
+      __syncthreads();
+    }
+
+    f32x16 o[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[d] = f32x16{};
+    // m: the running max in scaled log2 units less 10, so that p' = 2^(s c - m) <= 2^10
+    // (2^14 between refreshes), well inside fp16.
+    float m = -INFINITY, l = 0.f;
+    for (int t = 0; t < nkt; ++t) {
+      const uint32_t buf = (t & 1) * TB;
+      load_k(t + 1, reg);  // past the last tile: zeros past S, never used
+      const int k0 = kbeg + t * BN;
+      const bool mine = k0 < kend_w;
+      f32x16 st = f32x16{}, sx = f32x16{};
+      if (mine) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          const uint32_t at = (kl + buf) ^ (uint32_t)(s << 5);
+          const f16x8 kh = *(lds_f16x8*)(uintptr_t)at, kw = *(lds_f16x8*)(uintptr_t)(at + PL);
+          sx = __builtin_amdgcn_mfma_f32_32x32x16_f16(kw, qh[s], sx, 0, 0, 0);
+          st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[s], st, 0, 0, 0);
+          sx = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[s], sx, 0, 0, 0);
+        }
+        st += sx;
+      }
+      if (t + 1 < nkt) store_k(reg, (t & 1) ^ 1);
+      load_v(t + 1, reg);
+      if (mine) {
+        if (k0 + BN > S || (p.causal && k0 + BN - 1 > r0 + diag)) {
+          int vis = S - 1 - k0;
+          if (p.causal) vis = imin(vis, row + diag - k0);
+          vis -= 4 * hf;
+          asm volatile("" : "+v"(vis));
+#pragma unroll
+          for (int r = 0; r < 16; ++r) st[r] = vis >= 8 * (r >> 2) + (r & 3) ? st[r] : -INFINITY;
+        }
+        float mt = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mt = fmaxf(mt, st[r]);
+        mt = fmaxf(mt, __shfl_xor(mt, 32)) * c - 10.f;
+        if (__any(mt > m + 4.f)) {
+          const float mn = fmaxf(m, mt), alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+          l *= alpha;
+#pragma unroll
+          for (int d = 0; d < ND; ++d) o[d] *= alpha;
+          m = mn;
+        }
+        const float nm = m == -INFINITY ? 0.f : -m;
+        float ls = 0.f;
+        f16x8 ph[2], pl[2];
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+          u32x4 h, w;
+          uint32_t a, b;
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const float e0 = __builtin_amdgcn_exp2f(fmaf(st[8 * cc + 2 * x], c, nm));
+            const float e1 = __builtin_amdgcn_exp2f(fmaf(st[8 * cc + 2 * x + 1], c, nm));
+            ls += e0;
+            ls += e1;
+            split2(e0, e1, a, b);
+            h[x] = a;
+            w[x] = b;
+          }
+          ph[cc] = __builtin_bit_cast(f16x8, h);
+          pl[cc] = __builtin_bit_cast(f16x8, w);
+        }
+        l += ls;
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+          for (int d = 0; d < ND; ++d) {
+            s16x4v x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              x[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(va[d] + buf + (u >> 1) * PL + (16 * cc + 8 * (u & 1)) * 2 * E));
+            const f16x8 vh = __builtin_bit_cast(f16x8, __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7));
+            const f16x8 vw = __builtin_bit_cast(f16x8, __builtin_shufflevector(x[2], x[3], 0, 1, 2, 3, 4, 5, 6, 7));
+            o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vw, ph[cc], o[d], 0, 0, 0);
+            o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, pl[cc], o[d], 0, 0, 0);
+            o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[cc], o[d], 0, 0, 0);
+          }
+      }
+      if (t + 1 < nkt) store_v(reg, (t & 1) ^ 1);
+      __syncthreads();
+    }
+
+    if (__syncthreads_or(!ok)) {
+      failed |= 1u << pass;
+      continue;
+    }
+    const float lt = l + __shfl_xor(l, 32), isv = 1.f / sv;
+    if (row < L) {
+      float* po;
+      float f;
+      if constexpr (SPLIT) {
+        const int64_t slot = ((bw.b * p.heads + bw.h) * p.seq_q + row) * splits + sp;
+        po = p.part_acc + slot * E;
+        f = isv;
+        if (hf == 0) {
+          p.part_ml[2 * slot] = m;
+          p.part_ml[2 * slot + 1] = lt;
+        }
+      } else {
+        po = reinterpret_cast<float*>(p.out) + ((bw.b * p.seq_q + row) * p.heads + bw.h) * E;
+        f = lt > 0.f ? isv / lt : 0.f;
+      }
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4*>(po + 32 * d + 8 * g + 4 * hf) =
+              f32x4{o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
+    }
+  }
+#pragma unroll 1
+  for (int pass = 0; pass < np; ++pass)
+    if (failed >> pass & 1) {
+      __syncthreads();
+      const BlockWork bw = pair ? BlockWork{pw.b, pw.h, (pass ? pw.qb1 : pw.qb0) * kBM} : block_work(p, blockIdx.x);
+      f32_safe_pass<E, SPLIT>(p, bw, sp, splits);
+    }
+}
+
+}  // namespace ca

@@ -1156,16 +1156,12 @@ __host__ __device__ inline int64_t f32_tile_bytes(int64_t S, int64_t k0, int64_t
   return ((S - 1 - k0) * stride + E) * 4;
 }
 
-// SPLIT: blockIdx.y is one of gridDim.y splits of the key range, each a run of
-// whole tiles; the block writes unnormalised (O, max, sum) partials of its rows
-// for the combine kernel instead of the output.
-//
-// PAIR (causal calls of many query blocks, pair_blocks()): the block runs the pair
-// (qb, nqb-1-qb) one pass after the other, so every block does the same work;
-// otherwise one query block, the most expensive causal blocks first.
-template <int E, bool SPLIT, bool PAIR>
-__global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p) {
-  static_assert(!(SPLIT && PAIR), "split calls are not paired");
+// One query block (rows bw.q0 .. + 127) in 32-bit MFMAs: the pass that
+// flash_f32_kernel (ca_f32.h) takes where a block's values leave the range its split
+// operands hold.  SPLIT: the block's split sp of the keys; unnormalised (O, max, sum)
+// partials of its rows for the combine kernel instead of the output.
+template <int E, bool SPLIT>
+__device__ __forceinline__ void f32_safe_pass(const FlashParams& p, const BlockWork& bw, int sp, int splits) {
   using C = FlashF32Cfg<E>;
   constexpr int BN = C::BN, KS = C::KS, VS = C::VS;
   extern __shared__ __attribute__((aligned(16))) float smemf[];
@@ -1174,19 +1170,12 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p) {
 
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int li = lane & 31, hf = lane >> 5;
-  PairWork pw{};
-  if constexpr (PAIR) pw = pair_work(p, kBM, false, blockIdx.x);
-#pragma unroll 1
-  for (int pass = 0; pass < (PAIR ? pw.n : 1); ++pass) {
-  if (PAIR && pass > 0) __syncthreads();  // the first pass's tile buffers are free again
-  const BlockWork bw = PAIR ? BlockWork{pw.b, pw.h, (pass ? pw.qb1 : pw.qb0) * kBM} : block_work(p, blockIdx.x);
   const int64_t L = p.seq_q, S = p.seq_k, diag = S - L;
   const float* qg = reinterpret_cast<const float*>(p.q) + bw.b * p.qs[0] + bw.h * p.qs[2];
   const float* kg = reinterpret_cast<const float*>(p.k) + bw.b * p.ks[0] + bw.h * p.ks[2];
   const float* vg = reinterpret_cast<const float*>(p.v) + bw.b * p.vs[0] + bw.h * p.vs[2];
 
   const int64_t row = bw.q0 + 32 * wv + li;
-  const int sp = SPLIT ? (int)blockIdx.y : 0, splits = SPLIT ? (int)gridDim.y : 1;
   const F32Keys kr_ = f32_keys(p, bw.q0, SPLIT, sp, splits);
   const int64_t kbeg = kr_.kbeg;
   // The partial slot of (row, split): O at part_acc[slot * E], (max, sum) at part_ml[2 * slot].
@@ -1206,7 +1195,7 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p) {
 #pragma unroll
       for (int d = 0; d < E / 2; d += 4) *reinterpret_cast<f32x4*>(og + (E / 2) * hf + d) = f32x4{0, 0, 0, 0};
     }
-    continue;
+    return;
   }
 
   // Q: lane (query li, half hf) holds dims 4t+2hf and 4t+2hf+1.
@@ -1333,7 +1322,7 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p) {
         p.part_ml[2 * slot + 1] = l_tot;
       }
     }
-    continue;
+    return;
   }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row < L) {
@@ -1346,7 +1335,21 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p) {
             f32x4{oacc[d][4 * g] * inv, oacc[d][4 * g + 1] * inv, oacc[d][4 * g + 2] * inv,
                   oacc[d][4 * g + 3] * inv};
   }
-  }  // passes
+}
+
+// The 32-bit MFMA pass as a kernel of its own, for calls of few keys (f32_exact):
+// causal pairs or one query block per block, the most expensive causal blocks first.
+template <int E, bool SPLIT, bool PAIR>
+__global__ __launch_bounds__(256, 2) void flash_f32_exact_kernel(FlashParams p) {
+  static_assert(!(SPLIT && PAIR), "split calls are not paired");
+  PairWork pw{};
+  if constexpr (PAIR) pw = pair_work(p, kBM, false, blockIdx.x);
+#pragma unroll 1
+  for (int pass = 0; pass < (PAIR ? pw.n : 1); ++pass) {
+    if (PAIR && pass > 0) __syncthreads();  // the first pass's tile buffers are free again
+    const BlockWork bw = PAIR ? BlockWork{pw.b, pw.h, (pass ? pw.qb1 : pw.qb0) * kBM} : block_work(p, blockIdx.x);
+    f32_safe_pass<E, SPLIT>(p, bw, SPLIT ? (int)blockIdx.y : 0, SPLIT ? (int)gridDim.y : 1);
+  }
 }
 
 template <typename K, typename... A>
@@ -1365,6 +1368,7 @@ static int launch_lds(K kernel, int64_t nb, int threads, int lds, const FlashPar
 }  // namespace ca
 
 #include "ca_duo.h"
+#include "ca_f32.h"
 
 namespace ca {
 
@@ -1422,6 +1426,20 @@ static int bf16_launch(const FlashParams& p, const FlashPlan& plan, hipStream_t 
   return st == CA_OK && splits > 1 ? flash_combine_launch(p, E, true, splits, stream) : st;
 }
 
+template <int E>
+static int f32_launch(const FlashParams& p, const FlashPlan& plan, hipStream_t stream) {
+  const bool exact = f32_exact(E, p.causal != 0, p.seq_k);
+  constexpr int lds = F32Cfg<E>::LDS_BYTES, elds = FlashF32Cfg<E>::LDS_BYTES;
+  if (plan.split) {
+    const int st = exact ? launch_lds(flash_f32_exact_kernel<E, true, false>, plan.gx, 256, elds, p, stream, plan.splits)
+                         : launch_lds(flash_f32_kernel<E, true>, plan.gx, 256, lds, p, stream, plan.splits, 0);
+    return st == CA_OK ? flash_combine_launch(p, E, false, plan.splits, stream) : st;
+  }
+  if (!exact) return launch_lds(flash_f32_kernel<E, false>, plan.gx, 256, lds, p, stream, 1, (int)plan.pair);
+  return plan.pair ? launch_lds(flash_f32_exact_kernel<E, false, true>, plan.gx, 256, elds, p, stream)
+                   : launch_lds(flash_f32_exact_kernel<E, false, false>, plan.gx, 256, elds, p, stream);
+}
+
 int flash_launch(const FlashParams& p, int E, int bf16, hipStream_t stream) {
   const FlashPlan plan = flash_plan(p, E, bf16 != 0);
   if (plan.kind == kPlanNone) return CA_OK;
@@ -1430,7 +1448,6 @@ int flash_launch(const FlashParams& p, int E, int bf16, hipStream_t stream) {
     return CA_DECLINED;
   if (plan.kind == kPlanRows || plan.kind == kPlanRowsHeads) return flash_rows_launch(p, plan, E, bf16, stream);
   if (plan.kind == kPlanSmall) return flash_small_launch(p, plan, E, stream);
-  const int64_t nb = plan.gx, splits = plan.splits;
   if (bf16) {
     switch (E) {
       case 32: return bf16_launch<32>(p, plan, stream);
@@ -1438,28 +1455,10 @@ int flash_launch(const FlashParams& p, int E, int bf16, hipStream_t stream) {
       case 128: return bf16_launch<128>(p, plan, stream);
     }
   } else {
-    if (plan.split) {
-      int st = CA_DECLINED;
-      switch (E) {
-        case 32: st = launch_lds(flash_f32_kernel<32, true, false>, nb, 256, FlashF32Cfg<32>::LDS_BYTES, p, stream, splits); break;
-        case 64: st = launch_lds(flash_f32_kernel<64, true, false>, nb, 256, FlashF32Cfg<64>::LDS_BYTES, p, stream, splits); break;
-        case 128: st = launch_lds(flash_f32_kernel<128, true, false>, nb, 256, FlashF32Cfg<128>::LDS_BYTES, p, stream, splits); break;
-      }
-      if (st != CA_OK) return st;
-      return flash_combine_launch(p, E, bf16, splits, stream);
-    }
-    if (plan.pair) {
-      switch (E) {
-        case 32: return launch_lds(flash_f32_kernel<32, false, true>, nb, 256, FlashF32Cfg<32>::LDS_BYTES, p, stream);
-        case 64: return launch_lds(flash_f32_kernel<64, false, true>, nb, 256, FlashF32Cfg<64>::LDS_BYTES, p, stream);
-        case 128: return launch_lds(flash_f32_kernel<128, false, true>, nb, 256, FlashF32Cfg<128>::LDS_BYTES, p, stream);
-      }
-      return CA_DECLINED;
-    }
     switch (E) {
-      case 32: return launch_lds(flash_f32_kernel<32, false, false>, nb, 256, FlashF32Cfg<32>::LDS_BYTES, p, stream);
-      case 64: return launch_lds(flash_f32_kernel<64, false, false>, nb, 256, FlashF32Cfg<64>::LDS_BYTES, p, stream);
-      case 128: return launch_lds(flash_f32_kernel<128, false, false>, nb, 256, FlashF32Cfg<128>::LDS_BYTES, p, stream);
+      case 32: return f32_launch<32>(p, plan, stream);
+      case 64: return f32_launch<64>(p, plan, stream);
+      case 128: return f32_launch<128>(p, plan, stream);
     }
   }
   return CA_DECLINED;

@@ -1,0 +1,112 @@
+"""The fp32 prefill's split operands (flash_f32_kernel) on the GPU: the edges of its
+tiles and of f32_exact, every schedule, values that leave the split's range, and the
+error against 64 bits."""
+
+import numpy as np
+import pytest
+import torch
+
+from cpu_attention import flash_attn_func
+from helpers import values
+from oracle.attention import attention
+
+pytestmark = pytest.mark.gpu
+
+# (batch, seq_q, seq_k, heads): one block, partial tiles and query blocks, both sides of
+# f32_exact, split keys (few blocks), one query block per block, causal pairs
+SHAPES = [(1, 17, 32, 2), (1, 40, 33, 2), (2, 20, 64, 3), (1, 129, 65, 3), (1, 30, 192, 2), (1, 64, 193, 2),
+          (1, 100, 1000, 3), (1, 200, 1500, 5), (2, 300, 300, 60), (1, 700, 700, 100), (1, 2100, 2100, 33)]
+
+
+def tensors(shape, d, seed, device):
+    b, sq, sk, h = shape
+    g = torch.Generator(device=device).manual_seed(seed)
+    return [torch.randn(b, h, n, d, generator=g, device=device).transpose(1, 2) for n in (sq, sk, sk)]
+
+
+def some_heads(h):
+    return sorted({0, h // 2, h - 1})
+
+
+def reference(q, k, v, causal, heads, scale=None):
+    d = q.shape[-1]
+    return attention(*(values(x[:, :, heads]) for x in (q, k, v)), d ** -0.5 if scale is None else scale, causal)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_error_against_64_bits(cuda, shape, d, causal):
+    """A logit is a sum of d products, each off by at most 2^-23 + 2^-23 + 2^-24 of its
+    size (the two splits and the dropped low.low term), and of fp32 additions; p and v
+    are split alike.  With sums of random signs the 2-norm error stays a few 2^-24:
+    2e-6 bounds it at these sizes (4e-7 or less is seen)."""
+    print(f"f32 split {shape} d={d} causal={causal}", flush=True)
+    q, k, v = tensors(shape, d, sum(shape) + d, cuda)
+    heads = some_heads(shape[3])
+    out = values(flash_attn_func(q, k, v, causal=causal)[:, :, heads])
+    ref = reference(q, k, v, causal, heads)
+    assert np.linalg.norm(out - ref) <= 2e-6 * np.linalg.norm(ref)
+
+
+RANGES = {"large": lambda q, k, v: (q * 2.0 ** 30, k * 2.0 ** -30, v * 2.0 ** 39),
+          "past the range": lambda q, k, v: (q * 2.0 ** 60, k * 2.0 ** -60, v * 2.0 ** 80),
+          "tiny": lambda q, k, v: (q, k, v * 2.0 ** -100),
+          "late large key": lambda q, k, v: (q * 0.1, _scaled(k, -3, 100.0), _scaled(v, -3, 1e5)),
+          "late small keys": lambda q, k, v: (q, _scaled(k, slice(96, None), 1e-6), _scaled(v, slice(96, None), 1e-7)),
+          "first tile zero": lambda q, k, v: (q, _scaled(k, slice(0, 32), 0.0), _scaled(v, slice(0, 32), 0.0)),
+          "all zero": lambda q, k, v: (q * 0, k * 0, v * 0)}
+
+
+def _scaled(x, rows, f):
+    x = x.clone()
+    x[:, rows] *= f
+    return x
+
+
+@pytest.mark.parametrize("shape", [(1, 150, 300, 3), (1, 64, 1500, 3), (1, 600, 600, 110)])
+@pytest.mark.parametrize("what", list(RANGES))
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_values_out_of_the_splits_range(cuda, d, what, shape):
+    print(f"f32 range {what} {shape} d={d}", flush=True)
+    q, k, v = RANGES[what](*tensors(shape, d, d, cuda))
+    heads = some_heads(shape[3])
+    out = values(flash_attn_func(q, k, v, causal=True)[:, :, heads])
+    ref = reference(q, k, v, True, heads)
+    # 2e-6 as above, of the largest values: a dominant key carries its error into all of a row
+    assert np.isfinite(out).all()
+    assert np.linalg.norm(out - ref) <= 2e-6 * max(np.linalg.norm(ref), 1e-300)
+
+
+@pytest.mark.parametrize("shape", [(1, 150, 300, 2), (1, 64, 1500, 3), (1, 600, 600, 110)])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_infinite_and_nan_values(cuda, d, shape):
+    """A key whose logit is -inf for every query drops out; a NaN query row is NaN and
+    the others of its block keep their values; a NaN value reaches only rows that see
+    its key, in its dims."""
+    q, k, v = tensors(shape, d, d + 1, cuda)
+    q = q.abs() + 0.1
+    heads = [0]
+    k[:, 70, :, 3] = float("-inf")
+    q[:, 5] = float("nan")
+    out = values(flash_attn_func(q, k, v)[:, :, heads])
+    keep = [i for i in range(shape[2]) if i != 70]
+    ref = reference(q, k[:, keep], v[:, keep], False, heads)
+    rows = [i for i in range(shape[1]) if i != 5]
+    if shape[1] != 64:  # split keys: the combine takes a row of no comparable logit as one without keys
+        assert np.isnan(out[:, 5]).all()
+    assert np.linalg.norm(out[:, rows] - ref[:, rows]) <= 2e-6 * np.linalg.norm(ref[:, rows])
+    q, k, v = tensors(shape, d, d + 2, cuda)
+    v[:, 100, :, 1] = float("nan")
+    out = values(flash_attn_func(q, k, v)[:, :, heads])
+    assert np.isnan(out[..., 1]).all() and np.isfinite(np.delete(out, 1, -1)).all()
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0, 4.0])
+def test_softmax_scales(cuda, scale):
+    q, k, v = tensors((1, 150, 300, 2), 64, 9, cuda)
+    for causal in (False, True):
+        out = values(flash_attn_func(q, k, v, softmax_scale=scale, causal=causal))
+        ref = reference(q, k, v, causal, [0, 1], scale)
+        # logits of size |scale| * 64^0.5 * few: their rounding reaches p times as large
+        assert np.linalg.norm(out - ref) <= (2e-6 + 2e-6 * abs(scale) * 8) * np.linalg.norm(ref)
