@@ -21,7 +21,7 @@
 // 2^11); p by 2^10 (2^14 between two refreshes of the running max).  A block whose
 // values leave that range (a later tile's maximum 2^5 above or 2^14 below the first's, a
 // magnitude outside 2^+-40, inf or NaN) redoes the query block with the 32-bit MFMAs
-// (f32_safe_pass), so such inputs give what they gave before.
+// (ca_f32_pass.inc), so such inputs give what they gave before.
 //
 // Bound: the three MFMAs per product and the splitting of K and V tiles by every block
 // of 128 rows.  Measured back to back, before -> now: N=1 L=S=2048 H=32 E=128 causal 330
@@ -78,7 +78,7 @@ __device__ __forceinline__ float f32_scale(float mx, bool& ok) {
 }
 
 // Calls of few keys stay on the 32-bit MFMAs, which are closer to 64 bits there and no
-// slower (E=32 L=S=17: 4.3 against 5.4 us; E=32 L=S=200 causal error 1.9e-7 against
+// slower (E=32 L=S=17: 4.5 against 5.4 us; E=32 L=S=200 causal error 1.9e-7 against
 // 2.0e-7, non-causal from 48 keys
 // lower; E=64 L=S=32 causal 1.57e-7 against 1.68e-7, from 40 keys even).
 inline bool f32_exact(int E, bool causal, int64_t seq_k) {
@@ -370,12 +370,12 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pa
     }
   }
 #pragma unroll 1
-  for (int pass = 0; pass < np; ++pass)
-    if (failed >> pass & 1) {
-      __syncthreads();
-      const BlockWork bw = pair ? BlockWork{pw.b, pw.h, (pass ? pw.qb1 : pw.qb0) * kBM} : block_work(p, blockIdx.x);
-      f32_safe_pass<E, SPLIT>(p, bw, sp, splits);
-    }
+  for (int pass = 0; pass < np; ++pass) {
+    if (!(failed >> pass & 1)) continue;
+    __syncthreads();
+    const BlockWork bw = pair ? BlockWork{pw.b, pw.h, (pass ? pw.qb1 : pw.qb0) * kBM} : block_work(p, blockIdx.x);
+#include "ca_f32_pass.inc"
+  }
 }
 
 }  // namespace ca

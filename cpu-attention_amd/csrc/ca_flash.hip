@@ -1156,199 +1156,20 @@ __host__ __device__ inline int64_t f32_tile_bytes(int64_t S, int64_t k0, int64_t
   return ((S - 1 - k0) * stride + E) * 4;
 }
 
-// One query block (rows bw.q0 .. + 127) in 32-bit MFMAs: the pass that
-// flash_f32_kernel (ca_f32.h) takes where a block's values leave the range its split
-// operands hold.  SPLIT: the block's split sp of the keys; unnormalised (O, max, sum)
-// partials of its rows for the combine kernel instead of the output.
-template <int E, bool SPLIT>
-__device__ __forceinline__ void f32_safe_pass(const FlashParams& p, const BlockWork& bw, int sp, int splits) {
-  using C = FlashF32Cfg<E>;
-  constexpr int BN = C::BN, KS = C::KS, VS = C::VS;
-  extern __shared__ __attribute__((aligned(16))) float smemf[];
-  float* Ks = smemf;                 // [2][BN][KS]
-  float* Vs = smemf + 2 * C::LDS_K;  // [2][BN][VS]
-
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int li = lane & 31, hf = lane >> 5;
-  const int64_t L = p.seq_q, S = p.seq_k, diag = S - L;
-  const float* qg = reinterpret_cast<const float*>(p.q) + bw.b * p.qs[0] + bw.h * p.qs[2];
-  const float* kg = reinterpret_cast<const float*>(p.k) + bw.b * p.ks[0] + bw.h * p.ks[2];
-  const float* vg = reinterpret_cast<const float*>(p.v) + bw.b * p.vs[0] + bw.h * p.vs[2];
-
-  const int64_t row = bw.q0 + 32 * wv + li;
-  const F32Keys kr_ = f32_keys(p, bw.q0, SPLIT, sp, splits);
-  const int64_t kbeg = kr_.kbeg;
-  // The partial slot of (row, split): O at part_acc[slot * E], (max, sum) at part_ml[2 * slot].
-  const int64_t slot = ((bw.b * p.heads + bw.h) * L + row) * splits + sp;
-  const int nkt = kr_.nkt;
-  if (nkt == 0) {  // every row of the block sees no key of this range: exactly 0
-    if (SPLIT && row < L) {
-      float* pa = p.part_acc + slot * E;
-#pragma unroll
-      for (int d = 0; d < E / 2; d += 4) *reinterpret_cast<f32x4*>(pa + (E / 2) * hf + d) = f32x4{0, 0, 0, 0};
-      if (hf == 0) {
-        p.part_ml[2 * slot] = -INFINITY;
-        p.part_ml[2 * slot + 1] = 0.f;
-      }
-    } else if (row < L) {
-      float* og = reinterpret_cast<float*>(p.out) + ((bw.b * L + row) * p.heads + bw.h) * E;
-#pragma unroll
-      for (int d = 0; d < E / 2; d += 4) *reinterpret_cast<f32x4*>(og + (E / 2) * hf + d) = f32x4{0, 0, 0, 0};
-    }
-    return;
-  }
-
-  // Q: lane (query li, half hf) holds dims 4t+2hf and 4t+2hf+1.
-  float qr[E / 2];
-#pragma unroll
-  for (int t = 0; t < E / 4; ++t) {
-    u32x2 v = {0, 0};
-    if (row < L) v = *reinterpret_cast<const u32x2*>(qg + row * p.qs[1] + 4 * t + 2 * hf);
-    qr[2 * t] = __uint_as_float(v.x);
-    qr[2 * t + 1] = __uint_as_float(v.y);
-  }
-
-  const int64_t r0w = bw.q0 + 32 * wv;
-  const int64_t kend_w = p.causal ? min<int64_t>(S, r0w + 32 + diag) : S;
-
-  // Global -> register staging through buffer loads rebased at each tile (fixed
-  // per-lane offsets; rows past S read as zeros).
-  u32x4 kreg[C::CH], vreg[C::CH];
-  int koff[C::CH], voff[C::CH];
-#pragma unroll
-  for (int i = 0; i < C::CH; ++i) {
-    koff[i] = f32_tile_offset<E>(tid, i, p.ks[1]);
-    voff[i] = f32_tile_offset<E>(tid, i, p.vs[1]);
-  }
-  auto load_tile = [&](int t) {
-    const int64_t k0 = kbeg + (int64_t)t * BN;
-    const int64_t kbytes = f32_tile_bytes<E>(S, k0, p.ks[1]), vbytes = f32_tile_bytes<E>(S, k0, p.vs[1]);
-    const __amdgpu_buffer_rsrc_t kr = tile_rsrc(kg + k0 * p.ks[1], kbytes);
-    const __amdgpu_buffer_rsrc_t vr = tile_rsrc(vg + k0 * p.vs[1], vbytes);
-#pragma unroll
-    for (int i = 0; i < C::CH; ++i) {
-      kreg[i] = __builtin_amdgcn_raw_buffer_load_b128(kr, koff[i], 0, 0);
-      vreg[i] = __builtin_amdgcn_raw_buffer_load_b128(vr, voff[i], 0, 0);
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < C::CH; ++i) {
-      const int c = tid + 256 * i;
-      const int r = c / (E / 4), c4 = c % (E / 4);
-      float* kd = Ks + buf * C::LDS_K + r * KS + 4 * c4;
-      *reinterpret_cast<u32x2*>(kd) = u32x2{kreg[i].x, kreg[i].y};
-      *reinterpret_cast<u32x2*>(kd + 2) = u32x2{kreg[i].z, kreg[i].w};
-      *reinterpret_cast<u32x4*>(Vs + buf * C::LDS_V + r * VS + 4 * c4) = vreg[i];
-    }
-  };
-
-  f32x16 oacc[E / 32];
-#pragma unroll
-  for (int d = 0; d < E / 32; ++d) oacc[d] = f32x16{};
-  float m_run = -INFINITY, l_run = 0.f;
-  const float c = p.c;
-
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-  for (int t = 0; t < nkt; ++t) {
-    const int buf = t & 1;
-    load_tile(t + 1);  // past the last tile: never used (range-checked zeros past S)
-    const int64_t k0 = kbeg + (int64_t)t * BN;
-    if (k0 < kend_w) {
-      const float* kb = Ks + buf * C::LDS_K;
-      const float* vb = Vs + buf * C::LDS_V;
-      f32x16 st = f32x16{};
-#pragma unroll
-      for (int t4 = 0; t4 < E / 4; ++t4) {
-        const u32x2 a = *reinterpret_cast<const u32x2*>(kb + li * KS + 4 * t4 + 2 * hf);
-        st = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), qr[2 * t4], st, 0, 0, 0);
-        st = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), qr[2 * t4 + 1], st, 0, 0, 0);
-      }
-      const bool need_mask = (k0 + BN > S) || (p.causal && k0 + BN - 1 > r0w + diag);
-      const int64_t lim = r0w + li + diag;
-      float x[16];
-      float mt = -INFINITY;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float v = st[r] * c;
-        if (need_mask) {
-          const int64_t j = k0 + 8 * (r >> 2) + 4 * hf + (r & 3);
-          if (j >= S || (p.causal && j > lim)) v = -INFINITY;
-        }
-        x[r] = v;
-        mt = fmaxf(mt, v);
-      }
-      mt = fmaxf(mt, __shfl_xor(mt, 32));
-      const float m_new = fmaxf(m_run, mt);
-      const float mu = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - mu);
-      m_run = m_new;
-      float ls = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        x[r] = __builtin_amdgcn_exp2f(x[r] - mu);
-        ls += x[r];
-      }
-      l_run = l_run * alpha + ls;
-#pragma unroll
-      for (int d = 0; d < E / 32; ++d) oacc[d] *= alpha;
-      // O^T += V^T P^T, two keys per step: step r takes key 8(r/4)+4hf+r%4.
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = 8 * (r >> 2) + 4 * hf + (r & 3);
-#pragma unroll
-        for (int d = 0; d < E / 32; ++d)
-          oacc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[key * VS + 32 * d + li], x[r], oacc[d], 0, 0, 0);
-      }
-    }
-    store_tile(buf ^ 1);
-    __syncthreads();
-  }
-
-  const float l_tot = l_run + __shfl_xor(l_run, 32);
-  if constexpr (SPLIT) {
-    if (row < L) {
-      float* pa = p.part_acc + slot * E;
-#pragma unroll
-      for (int d = 0; d < E / 32; ++d)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<f32x4*>(pa + 32 * d + 8 * g + 4 * hf) =
-              f32x4{oacc[d][4 * g], oacc[d][4 * g + 1], oacc[d][4 * g + 2], oacc[d][4 * g + 3]};
-      if (hf == 0) {
-        p.part_ml[2 * slot] = m_run;
-        p.part_ml[2 * slot + 1] = l_tot;
-      }
-    }
-    return;
-  }
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (row < L) {
-    float* og = reinterpret_cast<float*>(p.out) + ((bw.b * L + row) * p.heads + bw.h) * E;
-#pragma unroll
-    for (int d = 0; d < E / 32; ++d)
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<f32x4*>(og + 32 * d + 8 * g + 4 * hf) =
-            f32x4{oacc[d][4 * g] * inv, oacc[d][4 * g + 1] * inv, oacc[d][4 * g + 2] * inv,
-                  oacc[d][4 * g + 3] * inv};
-  }
-}
-
-// The 32-bit MFMA pass as a kernel of its own, for calls of few keys (f32_exact):
-// causal pairs or one query block per block, the most expensive causal blocks first.
-template <int E, bool SPLIT, bool PAIR>
+// Calls of few keys (f32_exact in ca_f32.h).  PAIR (causal calls of many query blocks,
+// pair_blocks()): the block runs the pair (qb, nqb-1-qb) one pass after the other, so
+// every block does the same work; otherwise one query block, the most expensive causal
+// blocks first.
+template <int E, bool PAIR>
 __global__ __launch_bounds__(256, 2) void flash_f32_exact_kernel(FlashParams p) {
-  static_assert(!(SPLIT && PAIR), "split calls are not paired");
+  constexpr bool SPLIT = false;
   PairWork pw{};
   if constexpr (PAIR) pw = pair_work(p, kBM, false, blockIdx.x);
 #pragma unroll 1
   for (int pass = 0; pass < (PAIR ? pw.n : 1); ++pass) {
     if (PAIR && pass > 0) __syncthreads();  // the first pass's tile buffers are free again
     const BlockWork bw = PAIR ? BlockWork{pw.b, pw.h, (pass ? pw.qb1 : pw.qb0) * kBM} : block_work(p, blockIdx.x);
-    f32_safe_pass<E, SPLIT>(p, bw, SPLIT ? (int)blockIdx.y : 0, SPLIT ? (int)gridDim.y : 1);
+#include "ca_f32_pass.inc"
   }
 }
 
@@ -1428,16 +1249,16 @@ static int bf16_launch(const FlashParams& p, const FlashPlan& plan, hipStream_t 
 
 template <int E>
 static int f32_launch(const FlashParams& p, const FlashPlan& plan, hipStream_t stream) {
-  const bool exact = f32_exact(E, p.causal != 0, p.seq_k);
   constexpr int lds = F32Cfg<E>::LDS_BYTES, elds = FlashF32Cfg<E>::LDS_BYTES;
-  if (plan.split) {
-    const int st = exact ? launch_lds(flash_f32_exact_kernel<E, true, false>, plan.gx, 256, elds, p, stream, plan.splits)
-                         : launch_lds(flash_f32_kernel<E, true>, plan.gx, 256, lds, p, stream, plan.splits, 0);
-    return st == CA_OK ? flash_combine_launch(p, E, false, plan.splits, stream) : st;
+  if constexpr (E < 128) {
+    // Few enough keys for 32-bit MFMAs are too few to split.
+    if (f32_exact(E, p.causal != 0, p.seq_k) && !plan.split)
+      return plan.pair ? launch_lds(flash_f32_exact_kernel<E, true>, plan.gx, 256, elds, p, stream)
+                       : launch_lds(flash_f32_exact_kernel<E, false>, plan.gx, 256, elds, p, stream);
   }
-  if (!exact) return launch_lds(flash_f32_kernel<E, false>, plan.gx, 256, lds, p, stream, 1, (int)plan.pair);
-  return plan.pair ? launch_lds(flash_f32_exact_kernel<E, false, true>, plan.gx, 256, elds, p, stream)
-                   : launch_lds(flash_f32_exact_kernel<E, false, false>, plan.gx, 256, elds, p, stream);
+  if (!plan.split) return launch_lds(flash_f32_kernel<E, false>, plan.gx, 256, lds, p, stream, 1, (int)plan.pair);
+  const int st = launch_lds(flash_f32_kernel<E, true>, plan.gx, 256, lds, p, stream, plan.splits, 0);
+  return st == CA_OK ? flash_combine_launch(p, E, false, plan.splits, stream) : st;
 }
 
 int flash_launch(const FlashParams& p, int E, int bf16, hipStream_t stream) {
