@@ -23,9 +23,14 @@
 // magnitude outside 2^+-40, inf or NaN) redoes the query block with the 32-bit MFMAs
 // (ca_f32_pass.inc), so such inputs give what they gave before.
 //
+// Key groups (KG = 2): a second set of 4 waves on the same rows walks every other tile
+// and merges in LDS, as in flash_duo_kernel, for grids that give a CU one block: the
+// waves of one block do not cover each other's softmax and splitting (N=1 L=S=2048 H=32
+// E=128 causal, 256 pairs: 171 -> 139 us; L=S=4096 H=16 E=64 196 -> 143 us).
+//
 // Bound: the three MFMAs per product and the splitting of K and V tiles by every block
 // of 128 rows.  Measured back to back, before -> now: N=1 L=S=2048 H=32 E=128 causal 330
-// -> 171 us (201 TFLOP/s), N=1 L=S=4096 non-causal 2094 -> 947 us (290 TFLOP/s), N=4
+// -> 139 us (246 TFLOP/s), N=1 L=S=4096 non-causal 2094 -> 947 us (290 TFLOP/s), N=4
 // L=S=4096 H=32 E=64 causal 2266 -> 1136 us, N=8 L=S=512 H=16 E=64 81 -> 43 us, N=1 L=64
 // S=4096 H=8 E=64 30 -> 21 us.
 #pragma once
@@ -45,7 +50,10 @@ struct F32Cfg {
   static constexpr int PL = BN * E * 2;   // bytes of one plane (high or low halves) of a tile
   static constexpr int TB = 4 * PL;       // K high, K low, V high, V low
   static constexpr int CH = FlashF32Cfg<E>::CH;
-  static constexpr int LDS_BYTES = 2 * TB > FlashF32Cfg<E>::LDS_BYTES ? 2 * TB : FlashF32Cfg<E>::LDS_BYTES;
+  // Two tile buffers per key group, at least the 32-bit pass's buffers.
+  static constexpr int lds_bytes(int kg) { return 2 * kg * TB > FlashF32Cfg<E>::LDS_BYTES ? 2 * kg * TB : FlashF32Cfg<E>::LDS_BYTES; }
+  static constexpr int MERGE = E * 128 + 512;  // a wave's O, m and l for the merge of two groups
+  static_assert(4 * MERGE <= lds_bytes(2), "the merge fits the tile buffers");
 };
 
 __device__ __forceinline__ uint32_t f16_bits(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
@@ -85,17 +93,19 @@ inline bool f32_exact(int E, bool causal, int64_t seq_k) {
   return E == 32 ? seq_k <= (causal ? 192 : 32) : E == 64 && seq_k <= 32;
 }
 
-template <int E, bool SPLIT>
-__global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pair) {
+template <int E, int KG, bool SPLIT>
+__global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, int pair) {
   using C = F32Cfg<E>;
   constexpr int BN = C::BN, PL = C::PL, TB = C::TB, CH = C::CH, NS = E / 16, ND = E / 32;
   extern __shared__ __attribute__((aligned(1024))) char f32_smem[];
-  const int tid = threadIdx.x, lane = tid & 63;
+  static_assert(KG == 1 || !SPLIT, "split calls have one key group");
+  const int tid = threadIdx.x & 255, lane = tid & 63;  // thread of its key group
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8);
   const int li = lane & 31, hf = lane >> 5;
   PairWork pw{};
   if (pair) pw = pair_work(p, kBM, false, blockIdx.x);
-  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((const lds_void*)f32_smem);
+  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((const lds_void*)f32_smem) + grp * 2 * TB;
   const int sp = SPLIT ? (int)blockIdx.y : 0, splits = SPLIT ? (int)gridDim.y : 1;
   // LDS address of this thread's first staged chunk (8 bytes of halfs): K and V rows,
   // swizzled as the bf16 tiles; chunk i lies RI rows further (at E = 128 every other
@@ -123,7 +133,8 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pa
     const float* vg = reinterpret_cast<const float*>(p.v) + bw.b * p.vs[0] + bw.h * p.vs[2];
     const int r0 = (int)bw.q0 + 32 * wv, row = r0 + li;
     const F32Keys kr = f32_keys(p, bw.q0, SPLIT, sp, splits);
-    const int nkt = kr.nkt, kbeg = (int)kr.kbeg;
+    // Group g takes tiles g, g + KG, ...: its round t is tile t KG + g.
+    const int nkt = (kr.nkt + KG - 1) / KG, kbeg = (int)kr.kbeg;
     const int kend_w = p.causal ? imin(S, r0 + 32 + diag) : S;
 
     // Tiles: global -> registers (buffer loads rebased at each tile, zeros past the
@@ -132,7 +143,7 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pa
     const int koff = f32_tile_offset<E>(tid, 0, p.ks[1]), voff = f32_tile_offset<E>(tid, 0, p.vs[1]);
     const int kstep = (int)(RI * p.ks[1] * 4), vstep = (int)(RI * p.vs[1] * 4);
     auto load_one = [&](const float* g, int64_t stride, int off, int step, int t, u32x4 (&x)[CH]) __attribute__((always_inline)) {
-      const int64_t k0 = kbeg + (int64_t)t * BN;
+      const int64_t k0 = kbeg + ((int64_t)t * KG + grp) * BN;
       const __amdgpu_buffer_rsrc_t rs = tile_rsrc(g + k0 * stride, f32_tile_bytes<E>(S, k0, stride));
       asm volatile("" : "+v"(off));  // the chunks' offsets are added here, not kept
 #pragma unroll
@@ -234,7 +245,7 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pa
         mk = umax(mk, a);
         mv = umax(mv, b);
       }
-      uint32_t* w = reinterpret_cast<uint32_t*>(f32_smem);
+      uint32_t* w = reinterpret_cast<uint32_t*>(f32_smem + grp * 2 * TB);
       if (lane == 0) {
         w[2 * wv] = mk;
         w[2 * wv + 1] = mv;
@@ -265,8 +276,8 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pa
     for (int t = 0; t < nkt; ++t) {
       const uint32_t buf = (t & 1) * TB;
       load_k(t + 1, reg);  // past the last tile: zeros past S, never used
-      const int k0 = kbeg + t * BN;
-      const bool mine = k0 < kend_w;
+      const int k0 = kbeg + (t * KG + grp) * BN;
+      const bool mine = k0 < kend_w && (KG == 1 || t * KG + grp < kr.nkt);
       f32x16 st = f32x16{}, sx = f32x16{};
       if (mine) {
 #pragma unroll
@@ -345,7 +356,31 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pa
       failed |= 1u << pass;
       continue;
     }
-    const float lt = l + __shfl_xor(l, 32), isv = 1.f / sv;
+    float isv = 1.f / sv;
+    if constexpr (KG == 2) {
+      // Group 1's sums (in the values' own scale) go through LDS to group 0.
+      float* mb = reinterpret_cast<float*>(f32_smem + wv * C::MERGE) + lane;
+      if (grp == 1) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) mb[64 * (16 * d + r)] = o[d][r] * isv;
+        mb[64 * 16 * ND] = m;
+        mb[64 * 16 * ND + 64] = l;
+      }
+      __syncthreads();
+      if (grp == 1) continue;
+      const float m1 = mb[64 * 16 * ND], mn = fmaxf(m, m1), mu = mn == -INFINITY ? 0.f : mn;
+      const float w0 = __builtin_amdgcn_exp2f(m - mu), w1 = __builtin_amdgcn_exp2f(m1 - mu);
+      l = l * w0 + mb[64 * 16 * ND + 64] * w1;
+      m = mn;
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] = o[d][r] * (isv * w0) + mb[64 * (16 * d + r)] * w1;
+      isv = 1.f;
+    }
+    const float lt = l + __shfl_xor(l, 32);
     if (row < L) {
       float* po;
       float f;
@@ -369,6 +404,7 @@ __global__ __launch_bounds__(256, 2) void flash_f32_kernel(FlashParams p, int pa
               f32x4{o[d][4 * g] * f, o[d][4 * g + 1] * f, o[d][4 * g + 2] * f, o[d][4 * g + 3] * f};
     }
   }
+  if (grp == 1) return;  // the 32-bit pass takes one group (its barriers wait for the waves still running)
 #pragma unroll 1
   for (int pass = 0; pass < np; ++pass) {
     if (!(failed >> pass & 1)) continue;

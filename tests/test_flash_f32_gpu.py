@@ -13,9 +13,11 @@ from oracle.attention import attention
 pytestmark = pytest.mark.gpu
 
 # (batch, seq_q, seq_k, heads): one block, partial tiles and query blocks, both sides of
-# f32_exact, split keys (few blocks), one query block per block, causal pairs
+# f32_exact and of the two key groups' line, split keys (few blocks), one query block
+# per block, causal pairs with two key groups and with one
 SHAPES = [(1, 17, 32, 2), (1, 40, 33, 2), (2, 20, 64, 3), (1, 129, 65, 3), (1, 30, 192, 2), (1, 64, 193, 2),
-          (1, 100, 1000, 3), (1, 200, 1500, 5), (2, 300, 300, 60), (1, 700, 700, 100), (1, 2100, 2100, 33)]
+          (1, 70, 191, 2), (3, 330, 350, 20), (1, 100, 1000, 3), (1, 200, 1500, 5), (2, 300, 300, 60),
+          (1, 700, 700, 100), (1, 2048, 2048, 32), (1, 2100, 2100, 33)]
 
 
 def tensors(shape, d, seed, device):
