@@ -95,7 +95,14 @@ at::Tensor index_on(const at::Tensor& t, const at::Device& dev) {
   return t.device() == dev ? t : t.to(dev, /*non_blocking=*/true);
 }
 
-int64_t max_of(const at::Tensor& t) { return at::max(t).item<int64_t>(); }
+// The largest value of an index vector.  A short one on the GPU is copied over and
+// searched here: the copy is the synchronisation either way, and a reduction kernel
+// before it would be another launch (a decode call with the checks on: N=1 H=8 E=64, 256
+// keys 22.0 -> 18.8 us, N=1 H=32 E=128, 4095 keys 32.4 -> 29.4, N=128 31.0 -> 29.4).
+int64_t max_of(const at::Tensor& t) {
+  if (t.numel() == 1) return t.item<int64_t>();
+  return at::max(t.is_cuda() && t.nbytes() <= 4096 ? t.cpu() : t).item<int64_t>();
+}
 
 // torch's current stream on `dev` as a raw handle; nullptr with a Python error set.
 bool stream_of(const at::Device& dev, void** out) {
