@@ -172,8 +172,15 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
         top = max_abs16(max_abs16(top, hi.x), hi.y);
       }
       const uint32_t big = (top & 0xffff) > (top >> 16) ? top & 0xffff : top >> 16;
-      // fp16 0x2c00 = 2^-4: the wave's values reach within 2^-15 of the block's maximum.
-      ok &= !__any(big >= 0x7c00u) && (__any(big >= 0x2c00u) || !__any(big != 0u));
+      // fp16 0x2c00 = 2^-4: the wave's values reach within 2^-15 of the block's maximum,
+      // or all are 0 (the operands themselves: a high half of 0 may be an underflow).
+      ok &= !__any(big >= 0x7c00u);
+      if (!__any(big >= 0x2c00u)) {
+        uint32_t bits = 0;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) bits |= x[i].x | x[i].y | x[i].z | x[i].w;
+        ok &= !__any((bits & 0x7fffffffu) != 0u);
+      }
     };
     auto store_k = [&](const u32x4 (&x)[CH], int buf) __attribute__((always_inline)) { store_one(x, sk, kst + buf * TB, true); };
     auto store_v = [&](const u32x4 (&x)[CH], int buf) __attribute__((always_inline)) { store_one(x, sv, vst + buf * TB, false); };

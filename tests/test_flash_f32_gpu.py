@@ -80,6 +80,25 @@ def test_values_out_of_the_splits_range(cuda, d, what, shape):
     assert np.linalg.norm(out - ref) <= 2e-6 * max(np.linalg.norm(ref), 1e-300)
 
 
+@pytest.mark.parametrize("first", [2.0 ** 10, 0.0])
+@pytest.mark.parametrize("shape", [(1, 150, 300, 3), (1, 64, 1500, 3), (1, 600, 600, 110)])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_values_far_below_the_first_tiles(cuda, d, shape, first):
+    """The first tile's keys get no weight, and the values behind them lie below the
+    smallest fp16 at that tile's scale (or at the scale of a tile of zeros): they are
+    what the rows consist of, not zeros."""
+    print(f"f32 below the first tile's {first} {shape} d={d}", flush=True)
+    q, k, v = tensors(shape, d, d + 3, cuda)
+    q[..., 0], k[..., 0] = 40.0, 0.0
+    k[:, :32, :, 0] = -100.0  # a logit of -4000 d^-0.5: e^-353 of the others at most
+    v[:, :32] *= first
+    v[:, 32:] *= 2.0 ** -38
+    heads = some_heads(shape[3])
+    out = values(flash_attn_func(q, k, v)[:, :, heads])
+    ref = reference(q, k, v, False, heads)
+    assert np.linalg.norm(out - ref) <= 2e-6 * np.linalg.norm(ref)
+
+
 @pytest.mark.parametrize("shape", [(1, 150, 300, 2), (1, 64, 1500, 3), (1, 600, 600, 110)])
 @pytest.mark.parametrize("d", [32, 64, 128])
 def test_infinite_and_nan_values(cuda, d, shape):
