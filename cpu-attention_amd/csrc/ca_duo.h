@@ -424,6 +424,9 @@ __global__ __launch_bounds__(256 * KG, (DuoCfg<E, KG>::WAVES)) void flash_duo_ke
           mask(st[0], 0);
           m = row_max(st[0]) + (safe ? 0.f : P64Rows<E>::kMaxLift);
           nmu = m == -INFINITY ? 0.f : -m;
+          // No finite logit among the tile's visible keys: the max would be fixed at 0,
+          // and p of later logits far below 0 flush.
+          if (!safe) fine = m != -INFINITY || (p.causal && kbeg + grp * BN > r0 + li + diag);
           for (; t + 1 < nkt_w; t += 2) {
             body(std::integral_constant<int, 0>{}, t);
             body(std::integral_constant<int, 1>{}, t + 1);

@@ -42,3 +42,28 @@ def test_edges(cuda, shape, d, causal, gap):
             ke = min(sk, max(0, i + 1 + sk - sq)) if causal else sk
             ref.append(attention(qv[:, i:i + 1], kv[:, :ke], vv[:, :ke], d ** -0.5)[0, 0, 0] if ke else np.zeros(d))
         assert_close(torch.from_numpy(ov[0, rows, 0]), np.stack(ref), torch.bfloat16, paged=False)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("shape", [(1, 256, 900, 2), (1, 128, 2048, 2)])  # two key groups, split keys
+def test_first_tile_without_a_finite_logit(cuda, shape, d, causal):
+    """Every key of a group's or split's first tile has a logit of -inf, the others lie
+    near -200 log2 units: the row max is not fixed at 0, where their p would flush."""
+    b, sq, sk, h = shape
+    print(f"duo first tile -inf {shape} d={d} causal={causal}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(sk + d)
+    q, k, v = (torch.randn(b, h, n, d, generator=g, device=cuda).transpose(1, 2) for n in (sq, sk, sk))
+    q[..., :2], k[..., 0], k[..., 1] = 1.0, 0.0, -200 / 1.4427 * d ** 0.5
+    gone = [i for i in range(sk) if i // 64 in (1, 4)]
+    keep = [i for i in range(sk) if i // 64 not in (1, 4)]
+    k[:, gone, :, 0] = float("-inf")
+    q, k, v = (x.bfloat16() for x in (q, k, v))
+    out = values(flash_attn_func(q, k, v, causal=causal))
+    qv, kv, vv = values(q), values(k[:, keep]), values(v[:, keep])
+    rows = [0, 1, 63, 64, sq - 1]
+    ref = []
+    for i in rows:
+        n = sum(x <= i + sk - sq for x in keep) if causal else len(keep)
+        ref.append(attention(qv[:, i:i + 1], kv[:, :n], vv[:, :n], d ** -0.5)[0, 0])
+    assert_close(torch.from_numpy(out[0, rows]), np.stack(ref), torch.bfloat16, paged=False)
