@@ -21,7 +21,11 @@
 // Key groups (KG = 2): the block has a second set of 4 waves on the same rows; group
 // g walks tiles g, g + 2, ... through LDS buffers of its own, and the groups merge in
 // LDS at the end.  It halves the serial walk of a call whose blocks do not fill the
-// chip, with no partials in memory.
+// chip, with no partials in memory.  Both groups of a fast walk take p against the max
+// fixed at group 0's first tile, the pass's: one walk over all the tiles has that max
+// too, so P is rounded as there and the groups' sums add up whatever their sizes.  (A
+// max of each group's own can lie 2^126 from the other's while the rows' weight lies
+// in the lower one, whose merge weight flushes to 0.)
 // Split mode: the keys of each query block over gridDim.y blocks, partials merged by
 // the combine kernel (few query blocks over long keys).
 // Pairs (causal): query blocks (nqb - 1 - j, j) one after the other, so every block
@@ -42,15 +46,16 @@ struct DuoCfg {
   // the walk does not wait for its loads.
   static constexpr int NB = 2;
   static constexpr int GROUP_BYTES = 2 * NB * TB;  // LDS of one key group
-  static constexpr int LDS_BYTES = KG * GROUP_BYTES;
+  static constexpr int TILES = KG * GROUP_BYTES;
+  static constexpr int LDS_BYTES = TILES + (KG == 2 ? 4 * BM : 0);  // the rows' fixed max after the tiles
   static constexpr int NL = BN * CPR / (64 * NW);  // direct loads per thread and tile (K or V)
   static constexpr int STAGE_ROW = 2 * E + 16;     // output staging: bytes per row, padded
   static constexpr int MERGE = E * 128 + 512;      // a wave's O, m and l for the merge of two groups
   // Waves per SIMD the registers must allow: 3 where 168 registers hold a wave.
   static constexpr int WAVES = KG == 1 && E <= 64 ? 3 : 2;
   static_assert(NL * 64 * NW == BN * CPR, "the loads fill a tile exactly");
-  static_assert(NW * 32 * STAGE_ROW <= LDS_BYTES, "the staging fits the tile buffers");
-  static_assert(KG == 1 || (NW * MERGE <= LDS_BYTES && 32 * STAGE_ROW <= MERGE), "the merge fits the tile buffers");
+  static_assert(NW * 32 * STAGE_ROW <= TILES, "the staging fits the tile buffers");
+  static_assert(KG == 1 || (NW * MERGE <= TILES && 32 * STAGE_ROW <= MERGE), "the merge fits the tile buffers");
 };
 
 // LDS swizzles (tiles are unpadded: a direct load fills 64 consecutive chunks).
@@ -423,10 +428,20 @@ __global__ __launch_bounds__(256 * KG, (DuoCfg<E, KG>::WAVES)) void flash_duo_ke
           kb += TB;
           mask(st[0], 0);
           m = row_max(st[0]) + (safe ? 0.f : P64Rows<E>::kMaxLift);
+        }
+        if constexpr (KG == 2) {
+          if (!safe) {  // group 0's max for both (a wave without a tile there has none here)
+            float* first = reinterpret_cast<float*>(duo_smem + C::TILES) + 32 * wv + li;
+            if (grp == 0) *first = m;
+            __syncthreads();
+            m = *first;
+          }
+        }
+        if (nkt_w > 0) {
           nmu = m == -INFINITY ? 0.f : -m;
-          // No finite logit among the tile's visible keys: the max would be fixed at 0,
-          // and p of later logits far below 0 flush.
-          if (!safe) fine = m != -INFINITY || (p.causal && kbeg + grp * BN > r0 + li + diag);
+          // No finite logit among the first tile's visible keys: the max would be fixed
+          // at 0, and p of later logits far below 0 flush.
+          if (!safe) fine = m != -INFINITY || (p.causal && kbeg > r0 + li + diag);
           for (; t + 1 < nkt_w; t += 2) {
             body(std::integral_constant<int, 0>{}, t);
             body(std::integral_constant<int, 1>{}, t + 1);

@@ -1,6 +1,7 @@
 """flash_duo_kernel on the GPU at the edges of its tiles and of duo_plan's rules, with
 and without rows that take the safe walk, against the float64 oracle on sampled rows."""
 
+import math
 import random
 
 import numpy as np
@@ -67,3 +68,34 @@ def test_first_tile_without_a_finite_logit(cuda, shape, d, causal):
         n = sum(x <= i + sk - sq for x in keep) if causal else len(keep)
         ref.append(attention(qv[:, i:i + 1], kv[:, :n], vv[:, :n], d ** -0.5)[0, 0])
     assert_close(torch.from_numpy(out[0, rows]), np.stack(ref), torch.bfloat16, paged=False)
+
+
+# log2 units above the first tile's logits: a later key of the first tile's group (or
+# split) and a key in the first tile of the other one
+PEAKS = [(127.75, 126.25), (125, 127), (127.5, 127), (120, 118), (116, 128)]
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("peaks", PEAKS)
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_groups_of_far_apart_maxima(cuda, d, peaks, causal):
+    """Key 160 (tile 2, of key group 0) carries as much weight as key 70 (tile 1, group
+    1's first), both about 2^120 times the rest.  A max that each group fixed at its own
+    first tile would leave group 0's share a merge weight below the smallest fp32."""
+    far_apart(cuda, (1, 256, 900, 2), d, causal, {160: peaks[0], 70: peaks[1]})
+
+
+def far_apart(device, shape, d, causal, keys):
+    """Logits (log2 units) of 0 or a little more, and of keys[i] at key i."""
+    b, sq, sk, h = shape
+    print(f"duo far apart {shape} d={d} causal={causal} {keys}", flush=True)
+    g = torch.Generator(device=device).manual_seed(sk + d)
+    q, k, v = (0.1 * torch.randn(b, h, n, d, generator=g, device=device).transpose(1, 2) for n in (sq, sk, sk))
+    v = 10 * v
+    q[..., :2], k[..., :2] = 1.0, 0.0
+    for i, x in keys.items():
+        k[:, i, :, 0], k[:, i, :, 1] = int(x), x - int(x)
+    q, k, v = (x.bfloat16() for x in (q, k, v))
+    out = values(flash_attn_func(q, k, v, softmax_scale=math.log(2), causal=causal))
+    ref = attention(values(q), values(k), values(v), math.log(2), causal)
+    assert_close(torch.from_numpy(out), ref, torch.bfloat16, paged=False)
