@@ -500,9 +500,10 @@ __global__ __launch_bounds__(256 * KG, (DuoCfg<E, KG>::WAVES)) void flash_duo_ke
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[d][r] = o[d][r] * w0 + mb[64 * (16 * d + r)] * w1;
     }
-    const float lt = l + __shfl_xor(l, 32);
+    float lt = l + __shfl_xor(l, 32);
     if constexpr (SPLIT) {
       // The rows' partials for the combine: O unnormalised, m (scaled log2 units), l.
+      const float f = level_partial(m, lt);
       const int row = r0 + li;
       if (row < L) {
         const int64_t slot = (((int64_t)dw.b * p.heads + dw.h) * p.seq_q + row) * gridDim.y + blockIdx.y;
@@ -511,7 +512,7 @@ __global__ __launch_bounds__(256 * KG, (DuoCfg<E, KG>::WAVES)) void flash_duo_ke
         for (int d = 0; d < ND; ++d)
 #pragma unroll
           for (int q = 0; q < 4; ++q)
-            *reinterpret_cast<f32x4*>(po + 32 * d + 8 * q) = f32x4{o[d][4 * q], o[d][4 * q + 1], o[d][4 * q + 2], o[d][4 * q + 3]};
+            *reinterpret_cast<f32x4*>(po + 32 * d + 8 * q) = f32x4{o[d][4 * q] * f, o[d][4 * q + 1] * f, o[d][4 * q + 2] * f, o[d][4 * q + 3] * f};
         if (hf == 0) {
           p.part_ml[2 * slot] = m;
           p.part_ml[2 * slot + 1] = lt;

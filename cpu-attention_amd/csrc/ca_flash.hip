@@ -326,6 +326,20 @@ __device__ __forceinline__ float mask_key(float v, int vis, int key) {
   return v + __int_as_float(msk & (int)0xff800000u);
 }
 
+// A row's (O, m, l) partial for the combine kernel, which weighs the splits by their m
+// alone.  A fast walk's m lies 64 above its first tile's max and its sums reach 2^64, so
+// the split's weight is up to 2^64 above or below 2^m: two splits' m may lie past 2^126
+// apart, where the lower one's weight flushes to 0, while it holds most of the row.  The
+// exponent of l goes into m (l is 2^-7 .. 2^-6 then: sums over 64 splits of O stay within
+// V's size).  Returns the factor of O.
+__device__ __forceinline__ float level_partial(float& m, float& l) {
+  if (!(l > 0.f && l < INFINITY)) return 1.f;  // no visible key, or not finite
+  const float up = m + (float)((int)(__float_as_uint(l) >> 23) - 127 + 7), f = __builtin_amdgcn_exp2f(m - up);
+  m = up;
+  l *= f;
+  return f;
+}
+
 // State and key-tile step of the safe pass (one column block): 32 query rows of
 // one (batch, head), lane (query li, half hf), with a running max.
 template <int E>
@@ -823,7 +837,7 @@ struct P64Rows {
   static constexpr int kPartBytes = 32 * kPartRow;
 
   // The rows' partial for the combine (keys split over blocks): O^T unnormalised
-  // (fp32), the fixed max m (scaled log2 units) and l, at slot slot0 + row *
+  // (fp32), m (scaled log2 units) and l (level_partial), at slot slot0 + row *
   // splits of the workspace, staged through this wave's `stage` area as
   // store_staged stages the output (each store instruction writes 256 / E whole
   // rows).  A row that saw no key leaves m = -inf, l = 0, O = 0.
@@ -834,11 +848,12 @@ struct P64Rows {
     const int ch = lane % CPR, rr0 = lane / CPR;
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
-      const float lt = l[cb] + __shfl_xor(l[cb], 32);
+      float lt = l[cb] + __shfl_xor(l[cb], 32), mt = m[cb];
+      const float f = level_partial(mt, lt);
       const int rowl = r0 + 32 * cb + li;
       if (hf == 0 && rowl < a.L) {
         const int64_t slot = slot0 + (int64_t)rowl * splits;
-        pml[2 * slot] = m[cb];
+        pml[2 * slot] = mt;
         pml[2 * slot + 1] = lt;
       }
       char* rowp = stage + li * kPartRow;
@@ -847,7 +862,7 @@ struct P64Rows {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           *reinterpret_cast<f32x4*>(rowp + (32 * d + 8 * q + 4 * hf) * 4) =
-              f32x4{o[cb][d][4 * q], o[cb][d][4 * q + 1], o[cb][d][4 * q + 2], o[cb][d][4 * q + 3]};
+              f32x4{o[cb][d][4 * q] * f, o[cb][d][4 * q + 1] * f, o[cb][d][4 * q + 2] * f, o[cb][d][4 * q + 3] * f};
 #pragma unroll
       for (int k = 0; k < 32 / RPI; ++k) {
         const int rr = rr0 + RPI * k, row = r0 + 32 * cb + rr;

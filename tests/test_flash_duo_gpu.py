@@ -85,6 +85,17 @@ def test_groups_of_far_apart_maxima(cuda, d, peaks, causal):
     far_apart(cuda, (1, 256, 900, 2), d, causal, {160: peaks[0], 70: peaks[1]})
 
 
+# (1, 128, 2048): 8 splits of 256 keys; (1, 512, 6144): 7 of 896, at d = 128 on the 64-row kernel
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("peaks", PEAKS)
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("shape,key", [((1, 128, 2048, 2), 262), ((1, 512, 6144, 17), 902)])
+def test_splits_of_far_apart_maxima(cuda, shape, key, d, peaks, causal):
+    """As above, of two splits' partials: key 160 lies in tile 2 of split 0, `key` in the
+    first tile of split 1."""
+    far_apart(cuda, shape, d, causal, {160: peaks[0], key: peaks[1]})
+
+
 def far_apart(device, shape, d, causal, keys):
     """Logits (log2 units) of 0 or a little more, and of keys[i] at key i."""
     b, sq, sk, h = shape
@@ -96,6 +107,7 @@ def far_apart(device, shape, d, causal, keys):
     for i, x in keys.items():
         k[:, i, :, 0], k[:, i, :, 1] = int(x), x - int(x)
     q, k, v = (x.bfloat16() for x in (q, k, v))
-    out = values(flash_attn_func(q, k, v, softmax_scale=math.log(2), causal=causal))
-    ref = attention(values(q), values(k), values(v), math.log(2), causal)
+    out = flash_attn_func(q, k, v, softmax_scale=math.log(2), causal=causal)
+    q, k, v, out = (values(x[:, :, [0, h - 1]]) for x in (q, k, v, out))
+    ref = attention(q, k, v, math.log(2), causal)
     assert_close(torch.from_numpy(out), ref, torch.bfloat16, paged=False)
