@@ -652,17 +652,19 @@ struct P64Rows {
     }
   }
 
-  // Fixes each row's max at kMaxLift above tile 0's (every row that sees any key
-  // sees key 0), in scaled log2 units as the reference takes it.  The softmax is
+  // Fixes each row's max at kMaxLift above tile 0's (every row that sees any key of
+  // [kbeg, ..) sees key kbeg), in scaled log2 units as the reference takes it.  The softmax is
   // the same for any max; the lift only moves the window of logits the fixed max
   // serves exactly.  p of tile 0's largest logit is 2^-64, so p stays a normal
   // fp32 (and bf16) for logits down to 62 below it: smaller ones weigh less than
   // 2^-62 against that key and may flush to 0.  Upwards, a lane's sum of p over a
   // tile stays within the walk's 2^64 headroom for logits up to about 123 above
   // tile 0's max (64 without the lift); only rows whose logits outgrow that go
-  // through the safe pass.
+  // through the safe pass.  False: a row sees keys of tile 0, but no finite logit (the
+  // max would be fixed at 0, and p of later logits far below 0 flush).
   static constexpr float kMaxLift = 64.f;
-  __device__ __forceinline__ void fix_max(float c) {
+  __device__ __forceinline__ bool fix_max(const Bf16Pass& a, int kbeg) {
+    bool fine = true;
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
       float mx = -INFINITY;
@@ -670,9 +672,11 @@ struct P64Rows {
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[0][cb][kt][r]);
-      m[cb] = fmaxf(mx, __shfl_xor(mx, 32)) * c + kMaxLift;
+      m[cb] = fmaxf(mx, __shfl_xor(mx, 32)) * a.c + kMaxLift;
       nmu[cb] = m[cb] == -INFINITY ? 0.f : -m[cb];
+      fine &= m[cb] != -INFINITY || (a.causal && kbeg > r0 + 32 * cb + li + a.diag);
     }
+    return fine;
   }
 
   // Iteration t of the walk, as one stream in which every MFMA shares its issue
@@ -1064,7 +1068,7 @@ __global__ __launch_bounds__(256, 1) void flash_bf16_p64_kernel(FlashParams p) {
         w.template step<1, false, true, false>(Vs, kbuf(0), a.c, [] {});
         P64Rows<E>::mfma_guard();
         w.template apply_mask<0>(a, kbeg, 0);
-        w.fix_max(a.c);
+        bad = !w.fix_max(a, kbeg);
         bad |= !w.template step<0, false, true, true>(Vs, kbuf(1), a.c, loads);
         loads_landed_barrier<2 * NL>();
         // Tiles 1 .. nkt_w - 1: the P.V of the previous tile, the softmax of

@@ -70,6 +70,36 @@ def test_first_tile_without_a_finite_logit(cuda, shape, d, causal):
     assert_close(torch.from_numpy(out[0, rows]), np.stack(ref), torch.bfloat16, paged=False)
 
 
+# (shape, first tiles of its passes or splits, causal): two key groups, split keys, and at
+# d = 128 the 64-row kernel's unsplit blocks, its split keys and its causal pairs
+FIRSTS = [((1, 256, 900, 2), (0,), True), ((1, 128, 2048, 2), (0, 4), True), ((1, 256, 2560, 240), (0,), False),
+          ((1, 512, 6144, 17), (0, 14), False), ((1, 6144, 6144, 11), (0,), True)]
+
+
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("shape,tiles,causal", FIRSTS)
+def test_first_tile_of_a_walk_without_a_finite_logit(cuda, shape, tiles, causal, d):
+    """As above, of the tile that fixes the max of every walk."""
+    b, sq, sk, h = shape
+    print(f"first tile -inf {shape} d={d} causal={causal}", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(sk + d)
+    q, k, v = (torch.randn(b, h, n, d, generator=g, device=cuda).transpose(1, 2) for n in (sq, sk, sk))
+    q[..., :2], k[..., 0], k[..., 1] = 1.0, 0.0, -200 / 1.4427 * d ** 0.5
+    for t in tiles:
+        k[:, 64 * t:64 * t + 64, :, 0] = float("-inf")
+    q, k, v = (x.bfloat16() for x in (q, k, v))
+    out = flash_attn_func(q, k, v, causal=causal)
+    keep = [i for i in range(sk) if i // 64 not in tiles]
+    rows = [i for i in (0, 31, 64, 100, 255, 256, 3000, sq - 1) if i < sq and (not causal or i + sk - sq >= 64)]
+    for hh in (0, h - 1):
+        qv, kv, vv = values(q[:, rows, hh:hh + 1]), values(k[:, keep, hh:hh + 1]), values(v[:, keep, hh:hh + 1])
+        ref = []
+        for j, i in enumerate(rows):
+            n = sum(x <= i + sk - sq for x in keep) if causal else len(keep)
+            ref.append(attention(qv[:, j:j + 1], kv[:, :n], vv[:, :n], d ** -0.5)[0, 0, 0])
+        assert_close(out[0, rows, hh], np.stack(ref), torch.bfloat16, paged=False)
+
+
 # log2 units above the first tile's logits: a later key of the first tile's group (or
 # split) and a key in the first tile of the other one
 PEAKS = [(127.75, 126.25), (125, 127), (127.5, 127), (120, 118), (116, 128)]
