@@ -5,23 +5,48 @@
 // into two fp16 values, high = fp16(x) and low = fp16(x - high), which hold 23 of its 24
 // significant bits (24 where the low one needs at most 11), and a product takes three
 // 32x32x16 fp16 MFMAs with fp32 sums: high.high + high.low + low.high (the low.low term
-// is below 2^-24 of the product).  That is 96 instead of 512 cycles.  Probabilities,
-// their sums and the output stay fp32; P is split in the same way for P.V.
+// is below 2^-22 of the product, 2^-25 on average).  That is 96 instead of 512 cycles.
+// Probabilities, their sums and the output stay fp32; P is split in the same way for P.V.
 //
 // Precision.  Against 64 bits the split kernel is closer than the 32-bit MFMAs, whose
 // long chains of sums cost more than the splits (2-norm errors, N(0, 1) inputs, before
-// -> now): N=1 L=S=2048 H=32 E=128 causal 4.6e-7 -> 3.1e-7, L=S=4096 non-causal 1.2e-6
-// -> 7.8e-7, L=S=1024 H=16 E=64 causal 2.9e-7 -> 2.3e-7; with q 8 times larger (peaked
-// rows, E=64) 8.8e-7 -> 5.5e-7; with lognormal, shifted or per-channel scaled K and V it
-// is lower too.  Over few keys the chains are short and the splits would lose up to 45 %
-// (E=64 L=S=17 causal 1.2e-7 -> 1.7e-7): f32_exact leaves those calls to the 32-bit MFMAs.
+// -> now): N=1 L=S=2048 H=32 E=128 causal 4.6e-7 -> 2.7e-7, L=S=4096 non-causal 1.2e-6
+// -> 7.7e-7, L=S=1024 H=16 E=64 causal 2.8e-7 -> 2.3e-7; with q 8 times larger (peaked
+// rows) 1.6e-6 -> 6.9e-7, 2.0e-6 -> 9.3e-7, 1.0e-6 -> 5.0e-7; with lognormal V 4.8e-7 ->
+// 1.6e-7, 9.5e-7 -> 6.0e-7, 1.7e-7 -> 1.2e-7.  Over few keys the chains are short and
+// the splits would lose up to 45 % (E=64 L=S=17 causal 1.2e-7 -> 1.7e-7): f32_exact
+// leaves those calls to the 32-bit MFMAs.
 //
 // Range.  fp16 reaches from 2^-24 to 65504, so the operands are scaled by powers of two:
-// each Q row by its own maximum, K and V by that of the block's first tile, to [2^10,
-// 2^11); p by 2^10 (2^14 between two refreshes of the running max).  A block whose
-// values leave that range (a later tile's maximum 2^5 above or 2^14 below the first's, a
-// magnitude outside 2^+-40, inf or NaN) redoes the query block with the 32-bit MFMAs
-// (ca_f32_pass.inc), so such inputs give what they gave before.
+// each Q row by its own maximum, K and V by that of the range's first tile, to [2^10,
+// 2^11); p by 2^10 (2^14 between two refreshes of the running max).  Called q', k', v'
+// and p' then.  Below 2^-2 the low half is subnormal: an operand is off by up to a
+// quantum, 2^-25 (2^-25.8 rms), whatever its own size.  What that does to a row is
+// compared with what the row came out as, and a query block where it could cost more than
+// the 32-bit sums do is redone with the 32-bit MFMAs (ca_f32_pass.inc):
+//   logits  are off by c 2^-25.8 (|q'| + |k'|) in 2-norms, at most c 2^-21.3 times the
+//           larger of 2^11 and the largest |k'|; allowed is 2^-22.3, or X / 2 times that
+//           (a logit of X, in log2 units, is itself rounded by up to 2^-24 X): kF32Logit.
+//   O       is off in a row by 2^-25.8 times the root of sum p'^2 (V's quanta, in each
+//           dim) and by as much of the root of sum v'^2 (P's quanta, over all dims).  Its
+//           largest |O| has to be 2^23.8 times the first (sum p'^2 <= 2^14 sum p') and
+//           2^22.8 times the second: kF32RowSum, kF32RowKeys.  So rows whose weight lies
+//           on keys of much smaller values, or of none, are redone.
+//   columns of V must not hide behind larger ones: in every whole tile, of the 8 keys that
+//           a wave stages, one reaches 2^-3 (kF32Dense) in each column, whose quanta then
+//           stay below 2^-21.3 of it.  Columns that are 0 in the first tile must be 0 in
+//           all (padded head dims), and 8 keys of zeros pass (padded keys).  A column of
+//           zeros in some tiles only (a one-hot V, say) is redone: where the others have
+//           none, it consists of P's small values, which are quanta themselves.
+// (A single value far below both its row's and its column's others keeps its quantum's
+// error, small against theirs.)
+//   others: a K or V first tile of zeros or past the last key, a maximum outside 2^-40 ..
+//           2^40, a later tile's past 2^5 times the first's, inf or NaN.
+// What the first tile shows costs that tile alone (E=64 L=1024 S=8192 H=8, a V channel 1e4
+// times the others: 165 us, N(0, 1) 85, 32-bit MFMAs 156), the rest the walk.  Channels of
+// K 20 or of V 100 times the others, q 30 times larger or one value of 300 stay on the
+// split operands.  The checks cost 0 to 4 % (N=1 L=S=2048 H=32 E=128 causal 147.0 -> 147.8
+// us, N=8 L=S=512 H=16 E=64 35.7 -> 37.1, N=1 L=17 S=4096 H=8 E=128 27.6 -> 28.8).
 //
 // Key groups (KG = 2): a second set of 4 waves on the same rows walks every other tile
 // and merges in LDS, as in flash_duo_kernel, for grids that give a CU one block: the
@@ -50,14 +75,35 @@ struct F32Cfg {
   static constexpr int PL = BN * E * 2;   // bytes of one plane (high or low halves) of a tile
   static constexpr int TB = 4 * PL;       // K high, K low, V high, V low
   static constexpr int CH = FlashF32Cfg<E>::CH;
-  // Two tile buffers per key group, at least the 32-bit pass's buffers.
-  static constexpr int lds_bytes(int kg) { return 2 * kg * TB > FlashF32Cfg<E>::LDS_BYTES ? 2 * kg * TB : FlashF32Cfg<E>::LDS_BYTES; }
+  // Two tile buffers per key group, at least the 32-bit pass's buffers; after them a
+  // key group's exchange words: per wave the first tile's largest K and V magnitudes and
+  // the columns that its V rows are not all 0 in.
+  static constexpr int tiles(int kg) { return 2 * kg * TB > FlashF32Cfg<E>::LDS_BYTES ? 2 * kg * TB : FlashF32Cfg<E>::LDS_BYTES; }
+  static constexpr int XW = 8;  // words per wave
+  static constexpr int lds_bytes(int kg) { return tiles(kg) + kg * 4 * XW * 4; }
   static constexpr int MERGE = E * 128 + 512;  // a wave's O, m and l for the merge of two groups
-  static_assert(4 * MERGE <= lds_bytes(2), "the merge fits the tile buffers");
+  static_assert(4 * MERGE <= tiles(2), "the merge fits the tile buffers");
 };
 
 __device__ __forceinline__ uint32_t f16_bits(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ uint32_t umax(uint32_t a, uint32_t b) { return a > b ? a : b; }
+// The wave's combination of x in every lane: within rows of 16 lanes by rotations (no LDS
+// round trips, as shuffles take), then of the 4 rows.
+template <typename F>
+__device__ __forceinline__ uint32_t wave_fold(uint32_t x, F&& f) {
+  x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, false));  // row_ror:8
+  x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xf, 0xf, false));
+  x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x122, 0xf, 0xf, false));
+  x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xf, 0xf, false));
+  return f(f((uint32_t)__builtin_amdgcn_readlane((int)x, 0), (uint32_t)__builtin_amdgcn_readlane((int)x, 16)),
+           f((uint32_t)__builtin_amdgcn_readlane((int)x, 32), (uint32_t)__builtin_amdgcn_readlane((int)x, 48)));
+}
+__device__ __forceinline__ uint32_t wave_umax(uint32_t x) { return wave_fold(x, umax); }
+__device__ __forceinline__ float wave_fsum(float x) {
+  return __uint_as_float(wave_fold(__float_as_uint(x), [](uint32_t a, uint32_t b) __attribute__((always_inline)) {
+    return __float_as_uint(__uint_as_float(a) + __uint_as_float(b));
+  }));
+}
 // a and b, each as two fp16 values high + low (rounded to nearest even).
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
   const f16x2 h = {static_cast<_Float16>(a), static_cast<_Float16>(b)};
@@ -77,20 +123,42 @@ __device__ __forceinline__ int exp_of(float mx) { return (int)((__float_as_uint(
 
 constexpr int kF32Top = 10;  // the scaled block maximum lies in [2^10, 2^11)
 
-// The power of two that scales values up to mx to kF32Top, and whether the values are
-// ones the split holds: not past 2^40 (nor inf or NaN), nor, unless all are 0, below 2^-40.
+// The power of two that scales values up to mx to kF32Top; not ok: mx is 0, or outside
+// 2^-40 .. 2^40 (or inf or NaN).
 __device__ __forceinline__ float f32_scale(float mx, bool& ok) {
   const int e = exp_of(mx);
-  ok = mx == 0.f || (e >= -40 && e <= 40);
-  return mx == 0.f || !ok ? 1.f : __uint_as_float((uint32_t)(127 + kF32Top - e) << 23);
+  ok = e >= -40 && e <= 40;
+  return ok ? __uint_as_float((uint32_t)(127 + kF32Top - e) << 23) : 1.f;
 }
+
+// The limits of the quanta's part of the error (see Range above).
+constexpr float kF32Logit = 0.5f;       // c times the larger of 2^11 and the largest |k'|
+constexpr float kF32RowKeys = 1.f / 64;  // of the sum of all v' squared
+constexpr float kF32RowSum = 1024.f;    // of the sum of p'
+constexpr uint32_t kF32Dense = 0x3000;  // fp16 2^-3
+// p' = 2^(s c - m) is at most 2^10 at a refresh of m and 2^14 before the next.
+constexpr float kF32Lift = 10.f, kF32Slack = 4.f;
+
+// A wave's ballot over its staged chunks, one bit per 4 columns: lanes E / 4 apart hold
+// the same columns.
+template <int E>
+struct F32Cols {
+  static constexpr uint32_t ALL = E == 128 ? 0xffffffffu : (1u << (E / 4)) - 1;
+  __device__ __forceinline__ static uint32_t of(bool x) {
+    const uint64_t b = __ballot(x);
+    uint32_t r = (uint32_t)b | (uint32_t)(b >> 32);
+    if (E <= 64) r |= r >> 16;
+    if (E <= 32) r |= r >> 8;
+    return r & ALL;
+  }
+};
 
 // Calls of few keys stay on the 32-bit MFMAs, which are closer to 64 bits there and no
 // slower (E=32 L=S=17: 4.5 against 5.4 us; E=32 L=S=200 causal error 1.9e-7 against
-// 2.0e-7, non-causal from 48 keys
-// lower; E=64 L=S=32 causal 1.57e-7 against 1.68e-7, from 40 keys even).
+// 2.0e-7, non-causal from 48 keys lower; E=64 L=S=32 causal 1.57e-7 against 1.68e-7,
+// from 40 keys even), and calls without a whole key tile have to.
 inline bool f32_exact(int E, bool causal, int64_t seq_k) {
-  return E == 32 ? seq_k <= (causal ? 192 : 32) : E == 64 && seq_k <= 32;
+  return E == 32 ? seq_k <= (causal ? 192 : 32) : seq_k <= (E == 64 ? 32 : 31);
 }
 
 template <int E, int KG, bool SPLIT>
@@ -134,7 +202,8 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
     const int r0 = (int)bw.q0 + 32 * wv, row = r0 + li;
     const F32Keys kr = f32_keys(p, bw.q0, SPLIT, sp, splits);
     // Group g takes tiles g, g + KG, ...: its round t is tile t KG + g.
-    const int nkt = (kr.nkt + KG - 1) / KG, kbeg = (int)kr.kbeg;
+    int nkt = (kr.nkt + KG - 1) / KG;
+    const int kbeg = (int)kr.kbeg;
     const int kend_w = p.causal ? imin(S, r0 + 32 + diag) : S;
 
     // Tiles: global -> registers (buffer loads rebased at each tile, zeros past the
@@ -151,11 +220,29 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
     };
     auto load_k = [&](int t, u32x4 (&x)[CH]) __attribute__((always_inline)) { load_one(kg, p.ks[1], koff, kstep, t, x); };
     auto load_v = [&](int t, u32x4 (&x)[CH]) __attribute__((always_inline)) { load_one(vg, p.vs[1], voff, vstep, t, x); };
-    bool ok = true;  // every value so far is one the split operands hold
+    // Not ok: the split operands do not serve the query block (Range, above).  A range
+    // whose first tile is not whole has no tile to judge V's columns by.
+    bool ok = nkt == 0 || kbeg + (grp + 1) * BN <= S;
     float sk = 1.f, sv = 1.f;
-    // Splits this thread's staged values into the planes of a tile buffer.
+    uint32_t* xw = reinterpret_cast<uint32_t*>(f32_smem + C::tiles(KG)) + grp * 4 * C::XW;
+    bool zeros = false;  // some columns of the first V tile are all 0
+    uint32_t ktop = 0;   // this thread's largest |k'| (fp16 pairs; inf and NaN are largest)
+    float vsum = 0.f;    // per tile and column, its largest v' squared (CH times this bounds the sum)
+    // Whether some wave of the block has found the operands not to serve (word 6 or 7).
+    auto failing = [&](int word) __attribute__((always_inline)) {
+      const bool mine = __any(!ok);
+      if (lane == 0) xw[wv * C::XW + word] = mine;
+      __syncthreads();
+      const uint32_t* all = reinterpret_cast<const uint32_t*>(f32_smem + C::tiles(KG));
+      uint32_t any = 0;
+#pragma unroll
+      for (int w = 0; w < 4 * KG; ++w) any |= all[w * C::XW + word];
+      return __builtin_amdgcn_readfirstlane((int)any) != 0;
+    };
+    // Splits this thread's staged values into the planes of a tile buffer; the largest
+    // magnitudes of the high halves of columns 0 and 1 (top.x) and 2 and 3 (top.y).
     auto store_one = [&](const u32x4 (&x)[CH], float sc, uint32_t at0, bool k) __attribute__((always_inline)) {
-      uint32_t top = 0;
+      u32x2 top = {0, 0};
 #pragma unroll
       for (int i = 0; i < CH; ++i) {
         u32x2 hi, lo;
@@ -169,21 +256,45 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
         const uint32_t at = (k && E == 128 && (i & 1) ? at0 ^ 128u : at0) + i * RI * 2 * E;
         *(lds_u32x2*)(uintptr_t)at = hi;
         *(lds_u32x2*)(uintptr_t)(at + PL) = lo;
-        top = max_abs16(max_abs16(top, hi.x), hi.y);
+        const uint32_t h0 = hi.x, h1 = hi.y;
+        top = u32x2{max_abs16(top.x, h0), max_abs16(top.y, h1)};
       }
-      const uint32_t big = (top & 0xffff) > (top >> 16) ? top & 0xffff : top >> 16;
-      // fp16 0x2c00 = 2^-4: the wave's values reach within 2^-15 of the block's maximum,
-      // or all are 0 (the operands themselves: a high half of 0 may be an underflow).
-      ok &= !__any(big >= 0x7c00u);
-      if (!__any(big >= 0x2c00u)) {
+      return top;
+    };
+    auto store_k = [&](const u32x4 (&x)[CH], int buf) __attribute__((always_inline)) {
+      const u32x2 top = store_one(x, sk, kst + buf * TB, true);
+      ktop = max_abs16(max_abs16(ktop, top.x), top.y);
+    };
+    // The columns of V tile t that the wave's 8 rows hold a nonzero value in.
+    auto held = [&](const u32x4 (&x)[CH], uint32_t (&n)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
         uint32_t bits = 0;
 #pragma unroll
-        for (int i = 0; i < CH; ++i) bits |= x[i].x | x[i].y | x[i].z | x[i].w;
-        ok &= !__any((bits & 0x7fffffffu) != 0u);
+        for (int i = 0; i < CH; ++i) bits |= x[i][j];
+        n[j] = F32Cols<E>::of((bits & 0x7fffffffu) != 0);
       }
     };
-    auto store_k = [&](const u32x4 (&x)[CH], int buf) __attribute__((always_inline)) { store_one(x, sk, kst + buf * TB, true); };
-    auto store_v = [&](const u32x4 (&x)[CH], int buf) __attribute__((always_inline)) { store_one(x, sv, vst + buf * TB, false); };
+    auto store_v = [&](const u32x4 (&x)[CH], int t) __attribute__((always_inline)) {
+      const u32x2 top = store_one(x, sv, vst + (t & 1) * TB, false);
+      const uint32_t t0 = top.x, t1 = top.y;
+      vsum = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, t0), __builtin_bit_cast(f16x2, t0), vsum, false);
+      vsum = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, t1), __builtin_bit_cast(f16x2, t1), vsum, false);
+      if (kbeg + (t * KG + grp + 1) * BN > S) return;
+      const uint32_t r[4] = {F32Cols<E>::of((top.x & 0xffff) >= kF32Dense), F32Cols<E>::of((top.x >> 16) >= kF32Dense),
+                             F32Cols<E>::of((top.y & 0xffff) >= kF32Dense), F32Cols<E>::of((top.y >> 16) >= kF32Dense)};
+      if (__builtin_expect((r[0] & r[1] & r[2] & r[3]) == F32Cols<E>::ALL && !zeros, 1)) return;
+      uint32_t n[4];
+      held(x, n);
+      if ((n[0] | n[1] | n[2] | n[3]) == 0) return;  // 8 rows of zeros
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint32_t first = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) first |= xw[w * C::XW + 2 + j];
+        ok &= (((first & ~r[j]) | (n[j] & ~first)) & F32Cols<E>::ALL) == 0;
+      }
+    };
 
     u32x4 vreg0[CH];
     if (nkt > 0) {
@@ -214,12 +325,12 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
       // A negative softmax scale turns Q's sign instead, and a zero one zeroes Q, so
       // that c > 0: the running max is taken of the raw logits, and -inf * c is -inf.
       float sq = f32_scale(mx, fits);
-      ok &= __all(fits);
+      ok &= __all(fits || mx == 0.f);
       c = fabsf(p.c) / sq;
       sq = p.c < 0.f ? -sq : sq;
-      if (p.c == 0.f) {
+      if (p.c == 0.f || mx == 0.f) {  // logits of 0 for any small c > 0
         sq = 0.f;
-        c = 1.f;
+        c = 0x1p-60f;
       }
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
@@ -246,39 +357,40 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
           mk = umax(mk, a);
           mv = umax(mv, b);
         }
-#pragma unroll
-      for (int x = 32; x > 0; x >>= 1) {
-        const uint32_t a = __shfl_xor(mk, x), b = __shfl_xor(mv, x);
-        mk = umax(mk, a);
-        mv = umax(mv, b);
-      }
-      uint32_t* w = reinterpret_cast<uint32_t*>(f32_smem + grp * 2 * TB);
+      mk = wave_umax(mk);
+      mv = wave_umax(mv);
+      uint32_t n[4];
+      held(vreg0, n);
       if (lane == 0) {
-        w[2 * wv] = mk;
-        w[2 * wv + 1] = mv;
+        uint32_t* w = xw + wv * C::XW;
+        w[0] = mk;
+        w[1] = mv;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[2 + j] = n[j];
       }
       __syncthreads();
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
-        mk = umax(mk, w[2 * x]);
-        mv = umax(mv, w[2 * x + 1]);
+        mk = umax(mk, xw[x * C::XW]);
+        mv = umax(mv, xw[x * C::XW + 1]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) n[j] |= xw[x * C::XW + 2 + j];
       }
-      __syncthreads();
+      zeros = __any((n[0] & n[1] & n[2] & n[3]) != F32Cols<E>::ALL);
       bool fk, fv;
       sk = f32_scale(__uint_as_float(mk), fk);
       sv = f32_scale(__uint_as_float(mv), fv);
-      ok &= fk && fv;
       c /= sk;
+      ok &= fk && fv;
       store_k(reg, 0);
       store_v(vreg0, 0);
-      __syncthreads();
+      if (failing(6)) nkt = 0;  // the 32-bit pass without the walk first
     }
 
     f32x16 o[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) o[d] = f32x16{};
-    // m: the running max in scaled log2 units less 10, so that p' = 2^(s c - m) <= 2^10
-    // (2^14 between refreshes), well inside fp16.
+    // m: the running max in scaled log2 units less kF32Lift.
     float m = -INFINITY, l = 0.f;
     for (int t = 0; t < nkt; ++t) {
       const uint32_t buf = (t & 1) * TB;
@@ -311,8 +423,8 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
         float mt = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 16; ++r) mt = fmaxf(mt, st[r]);
-        mt = fmaxf(mt, __shfl_xor(mt, 32)) * c - 10.f;
-        if (__any(mt > m + 4.f)) {
+        mt = fmaxf(mt, __shfl_xor(mt, 32)) * c - kF32Lift;
+        if (__any(mt > m + kF32Slack)) {
           const float mn = fmaxf(m, mt), alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
           l *= alpha;
 #pragma unroll
@@ -355,11 +467,37 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
             o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, ph[cc], o[d], 0, 0, 0);
           }
       }
-      if (t + 1 < nkt) store_v(reg, (t & 1) ^ 1);
+      if (t + 1 < nkt) store_v(reg, t + 1);
       __syncthreads();
     }
 
-    if (__syncthreads_or(!ok)) {
+    {
+      // The row's largest |O|, its sum of p', and what all waves staged, against the limits.
+      uint32_t kt = wave_umax(umax(ktop & 0xffff, ktop >> 16));
+      const float vw = wave_fsum(vsum);
+      if (lane == 0) {
+        xw[wv * C::XW] = kt;
+        xw[wv * C::XW + 1] = __float_as_uint(vw);
+      }
+      __syncthreads();
+      float vs = 0.f, top = 0.f;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        kt = umax(kt, xw[x * C::XW]);
+        vs += __uint_as_float(xw[x * C::XW + 1]);
+      }
+      const float kv = static_cast<float>(__builtin_bit_cast(f16x2, umax(kt, 0x6800u)).x);  // 2^11 or more
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) top = fmaxf(top, fabsf(o[d][r]));
+      top = fmaxf(top, __shfl_xor(top, 32));
+      const float lt = l + __shfl_xor(l, 32);
+      if (row < L && lt != 0.f)
+        ok &= kt < 0x7c00u && vs < INFINITY && top * top >= fmaf(lt, kF32RowSum, vs * (CH * kF32RowKeys)) &&
+              c * kv <= kF32Logit * fmaxf(1.f, 0.5f * fabsf(m + kF32Lift));
+    }
+    if (failing(7)) {
       failed |= 1u << pass;
       continue;
     }

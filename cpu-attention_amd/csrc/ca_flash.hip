@@ -1269,12 +1269,10 @@ static int bf16_launch(const FlashParams& p, const FlashPlan& plan, hipStream_t 
 template <int E>
 static int f32_launch(const FlashParams& p, const FlashPlan& plan, hipStream_t stream) {
   constexpr int lds = F32Cfg<E>::lds_bytes(1), elds = FlashF32Cfg<E>::LDS_BYTES;
-  if constexpr (E < 128) {
-    // Few enough keys for 32-bit MFMAs are too few to split.
-    if (f32_exact(E, p.causal != 0, p.seq_k) && !plan.split)
-      return plan.pair ? launch_lds(flash_f32_exact_kernel<E, true>, plan.gx, 256, elds, p, stream)
-                       : launch_lds(flash_f32_exact_kernel<E, false>, plan.gx, 256, elds, p, stream);
-  }
+  // Few enough keys for 32-bit MFMAs are too few to split.
+  if (f32_exact(E, p.causal != 0, p.seq_k) && !plan.split)
+    return plan.pair ? launch_lds(flash_f32_exact_kernel<E, true>, plan.gx, 256, elds, p, stream)
+                     : launch_lds(flash_f32_exact_kernel<E, false>, plan.gx, 256, elds, p, stream);
   // Two key groups where a CU gets at most one block and the keys are enough to share:
   // L=S=200 H=20 E=32 N=2 12.1 -> 11.4 us, N=1 L=129 S=200 H=3 E=128 even, L=64 S=128 H=16
   // E=128 15.6 -> 16.1 us, L=100 S=70 10.0 -> 11.2 us.  With more blocks the CUs' second

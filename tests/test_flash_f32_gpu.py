@@ -2,6 +2,8 @@
 tiles and of f32_exact, every schedule, values that leave the split's range, and the
 error against 64 bits."""
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -97,6 +99,82 @@ def test_values_far_below_the_first_tiles(cuda, d, shape, first):
     out = values(flash_attn_func(q, k, v)[:, :, heads])
     ref = reference(q, k, v, False, heads)
     assert np.linalg.norm(out - ref) <= 2e-6 * np.linalg.norm(ref)
+
+
+def _channel(x, c, f):
+    x = x.clone()
+    x[..., c] *= f
+    return x
+
+
+def _logit(q, k, keys, x):
+    """Logits of x on top for those keys, 0 for the others."""
+    q, k = q.clone(), k.clone()
+    q[..., 0], k[..., 0] = 4.0, 0.0
+    k[:, keys, :, 0] = x / 4 * q.shape[-1] ** 0.5
+    return q, k
+
+
+def _sink(q, k, v, r):
+    return *_logit(q * 0.3, k, 40, math.log(k.shape[1] / r)), _scaled(v, 40, 0.0)
+
+
+def _one_hot(q, k, v, r):
+    d = v.shape[-1]
+    one = torch.eye(d, device=v.device)[torch.arange(v.shape[1], device=v.device) % d]
+    return *_logit(q * 0.3, k, slice(3, None, d), math.log(r)), one[None, :, None].expand_as(v)
+
+
+# what lies r below the rest, and how large a logit that takes
+SPREADS = {"a channel of v": (lambda q, k, v, r: (q, k, _channel(v, 5, r)), 0),
+           "the other channels of v": (lambda q, k, v, r: (q, k, _channel(v, 5, 1 / r)), 0),
+           "every other key of v": (lambda q, k, v, r: (q, k, _scaled(v, slice(0, None, 2), r)), 0),
+           "the keys of v that weigh": (lambda q, k, v, r: (*_logit(q, k, slice(1, None, 2), -60),
+                                                            _scaled(v, slice(0, None, 2), r)), 60),
+           "the first row of v": (lambda q, k, v, r: (q, k, _scaled(v, 0, r)), 0),
+           "a channel of k": (lambda q, k, v, r: (_channel(q, 3, 1 / r), _channel(k, 3, r), v), 0),
+           "a channel of q": (lambda q, k, v, r: (_channel(q, 3, r), _channel(k, 3, 1 / r), v), 0),
+           "every other key": (lambda q, k, v, r: (q, _scaled(k, slice(0, None, 2), r), v), 0),
+           "the weight of all but a key of zeros": (_sink, math.log),
+           "the weight of one channel's keys": (_one_hot, math.log)}
+
+
+@pytest.mark.parametrize("r", [1e-3, 1e-5, 1e-7, 1e-11])
+@pytest.mark.parametrize("shape", [(1, 150, 300, 2), (1, 64, 1500, 3), (1, 600, 600, 110)])
+@pytest.mark.parametrize("what", list(SPREADS))
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_values_of_very_different_size(cuda, d, what, shape, r):
+    """Small values beside large ones, r apart, that the large ones do not hide: every
+    row's and every channel's error in its own norm.  A row or channel alone sees less
+    averaging than the whole output, so 3e-6 (the 32-bit MFMAs: up to 1.8e-6); a logit x
+    is a sum of d products, whose roundings, of 2^-24 x each, reach p as they are."""
+    make, size = SPREADS[what]
+    print(f"f32 spread {what} {r} {shape} d={d}", flush=True)
+    heads = some_heads(shape[3])
+    q, k, v = make(*tensors(shape, d, d + 4, cuda), r)
+    x = size if isinstance(size, int) else abs(size(r / shape[2]))
+    tol = 3e-6 + x * d ** 0.5 * 2.0 ** -23
+    for causal in (False, True):
+        out = values(flash_attn_func(q, k, v, causal=causal)[:, :, heads])
+        ref = reference(q, k, v, causal, heads)
+        rows = (what != "the other channels of v") * np.linalg.norm(out - ref, axis=3) / np.linalg.norm(ref, axis=3)
+        channels = np.linalg.norm(out - ref, axis=1) / np.linalg.norm(ref, axis=1)
+        assert rows.max() <= tol and channels.max() <= tol, (rows.max(), channels.max(), tol)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("shape", [(1, 40, 31, 3), (1, 40, 5, 3), (1, 17, 32, 2), (2, 33, 60, 3), (1, 40, 2049, 3),
+                                   (1, 300, 260, 30)])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_a_channel_in_few_keys(cuda, d, shape, causal):
+    """No whole key tile, one and a part of one, a split that holds a part alone, and
+    more rows than keys."""
+    q, k, v = tensors(shape, d, d + 6, cuda)
+    v = _channel(v, 5, 1e-7)
+    heads = some_heads(shape[3])
+    out, ref = values(flash_attn_func(q, k, v, causal=causal)[:, :, heads]), reference(q, k, v, causal, heads)
+    channels = np.linalg.norm(out - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert channels.max() <= 3e-6, channels.max()
 
 
 @pytest.mark.parametrize("shape", [(1, 150, 300, 2), (1, 64, 1500, 3), (1, 600, 600, 110)])
