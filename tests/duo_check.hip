@@ -8,6 +8,7 @@
 // hit the chunks that the loads filled.
 //
 // Input lines and --plant as geom_check.hip.  Output: "ok <taken> <accesses>".
+// --plans: instead, per line "<key groups, 0: the 64-row kernel> <splits> <pairs>".
 #include <stdio.h>
 #include <string.h>
 
@@ -79,6 +80,14 @@ static bool layout() {
 }
 
 template <int E>
+static void print_plan(const FlashParams& p) {
+  const FlashPlan plan = flash_plan(p, E, true);
+  if (plan.kind != kPlanBf16) return (void)puts("other route");
+  const DuoPlan d = duo_plan(p, E, plan);
+  printf("%d %d %d\n", d.kg, (int)(d.kg ? d.splits : plan.splits), d.kg ? d.pair : plan.pair);
+}
+
+template <int E>
 static bool check(const FlashParams& p, bool& taken) {
   const FlashPlan plan = flash_plan(p, E, true);
   if (plan.kind != kPlanBf16) return true;
@@ -131,6 +140,7 @@ static bool check(const FlashParams& p, bool& taken) {
 
 int main(int argc, char** argv) {
   g_plant = argc > 1 && !strcmp(argv[1], "--plant");
+  const bool plans = argc > 1 && !strcmp(argv[1], "--plans");
   long long n = 0, E, bf, causal, batch, sq, sk, h, qs[3], ks[3], vs[3];
   while (scanf("%lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lld %lld", &E, &bf, &causal,
                &batch, &sq, &sk, &h, &qs[0], &qs[1], &qs[2], &ks[0], &ks[1], &ks[2], &vs[0], &vs[1], &vs[2]) == 16) {
@@ -138,11 +148,15 @@ int main(int argc, char** argv) {
     p.batch = batch; p.seq_q = sq; p.seq_k = sk; p.heads = h; p.causal = (int)causal;
     for (int i = 0; i < 3; ++i) { p.qs[i] = qs[i]; p.ks[i] = ks[i]; p.vs[i] = vs[i]; }
     bool taken = false;
+    if (plans) {
+      E == 32 ? print_plan<32>(p) : E == 64 ? print_plan<64>(p) : print_plan<128>(p);
+      continue;
+    }
     if (bf && !(E == 32 ? check<32>(p, taken) : E == 64 ? check<64>(p, taken) : check<128>(p, taken))) {
       printf("FAIL E=%lld causal=%lld N=%lld L=%lld S=%lld H=%lld: %s\n", E, causal, batch, sq, sk, h, g_fail);
       return 1;
     }
     n += taken;
   }
-  printf("ok %lld %lld\n", n, g_checks);
+  if (!plans) printf("ok %lld %lld\n", n, g_checks);
 }

@@ -17,6 +17,9 @@ EDGES = [(1, 300, 512, 3), (1, 300, 513, 3), (1, 130, 577, 3), (1, 384, 640, 85)
          (1, 700, 700, 60), (1, 767, 767, 45), (1, 2112, 2112, 17), (3, 300, 300, 60), (1, 2050, 2050, 31),
          (1, 70, 4100, 3), (2, 500, 3000, 8), (1, 512, 2560, 21), (1, 512, 4096, 42), (1, 512, 6144, 17),
          (1, 700, 300, 50), (1, 1000, 2000, 40), (1, 1000, 1999, 40), (9, 50, 50, 130)]
+# E = 128 calls on the 64-row kernel: (shape, causal, splits, pairs)
+P64 = [((1, 6144, 6144, 11), True, 1, 1), ((1, 6150, 6200, 11), True, 1, 1), ((1, 250, 2570, 240), False, 1, 0),
+       ((1, 250, 2570, 240), True, 1, 0), ((1, 500, 6150, 17), False, 7, 0), ((1, 500, 6150, 17), True, 7, 0)]
 
 
 @pytest.fixture(scope="module")
@@ -43,3 +46,11 @@ def test_every_access_inside_its_tensor(checker):
 def test_a_planted_window_mistake_is_caught(checker):
     r = run(checker, [line(64, True, True, 1, 257, 513, 8)], "--plant")
     assert r.returncode == 1 and "FAIL" in r.stdout, r.stdout
+
+
+def test_calls_on_the_64_row_kernel(checker):
+    """The shapes of test_flash_p64_gpu.py run what that test is about."""
+    r = run(checker, [line(128, True, causal, *shape) for shape, causal, _, _ in P64], "--plans")
+    assert r.stdout.splitlines() == [f"0 {splits} {pairs}" for _, _, splits, pairs in P64], r.stdout
+    r = run(checker, [line(e, True, c, *s) for e in (32, 64) for s, c, _, _ in P64], "--plans")
+    assert not any(x.startswith("0") for x in r.stdout.splitlines()), r.stdout

@@ -153,10 +153,11 @@ def test_cfg4_cross_shape(cuda):
 def test_cfg4_prefill_full_size_sampled(cuda):
     """BASELINE cfg4: N=4 L=S=4096 H=32 E=128 causal bf16, q/k/v strided chunks of a
     fused [N*L, 3*H*E] projection.  The whole output is computed; the float64 oracle
-    checks every one of the 128 (batch, head) pairs, on one row of each 256-row
-    query block (a different offset per pair and block, so both passes of every
-    causal pair, every wave's rows and every block of the XCD schedule are seen)
-    and on the first and last rows, plus tile and block edges of a few pairs."""
+    checks every one of the 128 (batch, head) pairs, on one row of every 256 (a
+    different offset per pair and place, so that over the pairs every 128-row query
+    block, both passes of the causal pairs, every wave's rows and every block of the
+    XCD schedule are seen) and on the first and last rows, plus tile and block edges
+    of a few pairs."""
     N, L, H, E = 4, 4096, 32, 128
     g = torch.Generator(device=cuda).manual_seed(4)
     qkv = torch.randn(N * L, 3 * H * E, generator=g, device=cuda).to(torch.bfloat16)
@@ -211,21 +212,21 @@ def test_logits_outgrowing_the_first_tile(cuda, d, causal, gap):
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("bad_pass", [0, 1])
 def test_safe_pass_for_one_pass_of_a_causal_pair(cuda, d, bad_pass):
-    """A causal call of two 256-row query blocks runs as one pair in one bf16 block:
-    pass 0 (rows 256-511), then pass 1 (rows 0-255).  Only one of the two passes
-    holds rows whose logits outgrow the fast walk's fixed max; the block redoes
-    exactly those after both passes and keeps the other pass's fast results."""
+    """A causal call of four 128-row query blocks per head runs as two pairs, (3, 0) and
+    (2, 1): the high block first, then the low one.  Only one of the two passes of a
+    pair holds rows whose logits outgrow the fast walk's fixed max: the block walks
+    that pass again with a running max and keeps the other's fast results."""
     g = torch.Generator().manual_seed(12 + bad_pass)
-    b, L, h = 1, 512, 130  # 260 query blocks: paired
+    b, L, h = 1, 512, 130  # 520 query blocks of 128 rows: paired
     q = torch.randn(b, L, h, d, generator=g) * 0.5 + 1.0
     k = torch.randn(b, L, h, d, generator=g) * 0.5
     # a key whose logits sit about 180 log2 units above the first tile's max (past
     # the ~123 that the fast walk's fixed max and 2^64 headroom serve)
     big = 184 / (1.4427 * d ** 0.5)
     if bad_pass == 0:
-        k[:, 400] = big  # seen only by rows >= 400 (pass 0)
+        k[:, 400] = big  # seen only by rows >= 400 (query block 3, pass 0 of its pair)
     else:
-        k[:, 200] = big  # seen by every row >= 200: rows of pass 0 get q < 0 for it
+        k[:, 200] = big  # seen by every row >= 200: rows from 256 on get q < 0 for it, so query block 1 (pass 1) alone
         q[:, 256:] = -q[:, 256:]
     q, k = q.bfloat16().to(cuda), k.bfloat16().to(cuda)
     v = torch.randn(b, L, h, d, generator=g).bfloat16().to(cuda)
@@ -242,13 +243,13 @@ def test_every_wave_of_a_block_failing_the_walk(cuda, d, causal, sq, h):
     """Key 100 sits about 180 log2 units above every row's first-tile max (the fast
     walk serves ~123), so every wave whose rows see it fails the walk's headroom
     from tile 1 on, and
-    whole blocks redo their rows in the safe pass.  Causal, 1536 rows: the pair
-    (rows 1280-1535, rows 0-255) fails all of its first pass and part of its second
-    (whose first wave never sees key 100).  Non-causal, 600 rows over 1536 keys:
-    every full block fails; the last block's waves past row 599 do not.  With 2
-    heads the query blocks are few, so their keys are split over blocks (the safe
-    pass writes partials); with 44 or 86 heads they fill the chip (pairs when
-    causal, one block per query block otherwise)."""
+    whole blocks walk again with a running max.  Causal, 1536 rows: the pair (rows
+    1408-1535, rows 0-127) fails all of its first pass and the last wave of its second
+    (the others never see key 100).  Non-causal, 600 rows over 1536 keys: every full
+    block fails; the last block's waves past row 599 do not.  With 2 heads the query
+    blocks are few, so their keys are split over blocks (the second walk writes
+    partials); with 44 or 86 heads they fill the chip (pairs when causal, one block
+    per query block otherwise)."""
     g = torch.Generator().manual_seed(13)
     b = 1
     sk = 1536
@@ -273,18 +274,15 @@ def test_every_wave_of_a_block_failing_the_walk(cuda, d, causal, sq, h):
 def test_causal_block_schedules(cuda, d, b, sq, sk, h, dtype):
     """The causal block schedules, each checked on a few heads: query-block pairs
     (qb, nqb-1-qb) in one block when unpaired blocks would leave the chip
-    unevenly loaded, else one block per query block.  bf16 (256 rows per query
-    block) pairs past 256: 1 x 130 x 3 = 390 (two pairs and one lone block per
-    head) and 2 x 48 x 3 = 288 (more keys than rows) pair; 16 blocks over 400 keys
-    (too few keys to split) and 256 at L = 2048 do not.  fp32 (128 rows) pairs
-    from 1024, or from 512 with fewer than twice as many keys as rows: 650, 576
-    and 512 at L = S = 2048 pair (odd and even counts per head); 32, and 512 over
-    4096 keys, do not.  64 bf16 query blocks at L = S = 1024 run unsplit (causal
-    triangle); the same call in fp32 (128 query blocks) splits its keys.  Fewer
-    bf16 query blocks over at least 1024 keys split (32 at L = S = 2048: 8 splits;
-    60 at L = S = 1500: 4), over 512 keys they do not; 64 to 127 split over 2048
-    keys or more (64 at L = S = 4096: 4 splits), not below (120 at L = S = 1500),
-    causal or not; 128 split in two over 4096 keys or more."""
+    unevenly loaded, else one block per query block.  bf16, 128-row query blocks
+    (duo_plan): past 512 of them pairs (1 x 130 x 5 = 650, odd per head, and 2 x 48 x
+    6 = 576 with more keys than rows); 512 with as many keys as rows (L = 2048) pairs
+    with two key groups, over 4096 keys one block per query block at d = 64 and the
+    64-row kernel at d = 128; up to 256 two key groups (1024, 16 heads; 1500, 10 and 20;
+    4096, 8), over at most 512 keys one (400, 8; 512, 16), or 4 splits of the keys
+    (2048 and 4096, 4 heads).  fp32 (128 rows) pairs from 1024, or from 512 with fewer
+    than twice as many keys as rows: 650, 576 and 512 at L = S = 2048 pair (odd and
+    even counts per head); 512 over 4096 keys do not, and fewer split their keys."""
     g = torch.Generator().manual_seed(40 + h)
     q = torch.randn(b, sq, h, d, generator=g).to(dtype).to(cuda)
     k, v = (torch.randn(b, sk, h, d, generator=g).to(dtype).to(cuda) for _ in range(2))
@@ -298,7 +296,7 @@ def test_causal_block_schedules(cuda, d, b, sq, sk, h, dtype):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_causal_pairs_with_rows_without_keys(cuda, dtype):
     """Causal pairs whose low query blocks see no key: 2304 rows over 1024 keys, 32
-    heads (288 bf16 / 576 fp32 query blocks, both paired).  Rows below 1280 are
+    heads (576 query blocks of 128 rows, paired in both types).  Rows below 1280 are
     exactly 0, written by the passes that have no key tile."""
     g = torch.Generator().manual_seed(50)
     b, sq, sk, h, d = 1, 2304, 1024, 32, 64
@@ -333,9 +331,9 @@ def test_split_keys(cuda, d, causal, shape, dtype):
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("b,sq,sk,h", [(2, 600, 600, 8), (1, 512, 512, 8), (1, 768, 768, 4), (1, 1000, 1000, 2)])
 def test_short_key_split_rule(cuda, d, b, sq, sk, h):
-    """bf16 non-causal calls under 1024 keys (fewer than twice as many keys as
-    rows): from 16 query blocks unsplit (48 and 16 here), below it their keys split
-    over blocks (12 and 8)."""
+    """bf16 non-causal calls around 1024 keys (fewer than twice as many keys as rows):
+    two key groups per block (2 x 600, 8 heads; 768, 4), one over 512 keys, and keys
+    split over blocks (1000 keys, 2 heads: 16 query blocks in 4 splits)."""
     print(f"short-key split rule b={b} sq={sq} sk={sk} h={h} d={d}", flush=True)
     run(b, sq, sk, h, d, torch.bfloat16, False, 61 + sq, cuda)
 
