@@ -38,7 +38,7 @@ template <int E, int KG>
 struct DuoCfg {
   static constexpr int NW = 4;       // waves per key group
   static constexpr int BM = 32 * NW; // query rows per block
-  static constexpr int BN = 64;      // keys per tile
+  static constexpr int BN = kTileKeys;
   static constexpr int CPR = E / 8;  // 16-byte chunks per row
   static constexpr int TB = BN * E * 2;  // bytes per tile buffer (no padding: swizzled)
   // Two buffers each for K and V: K(t + 2) and V(t + 1) load during tile t.  Three
@@ -427,7 +427,7 @@ __global__ __launch_bounds__(256 * KG, (DuoCfg<E, KG>::WAVES)) void flash_duo_ke
             st[0][q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kread(kb, q), qr[q >> 1], q < 2 ? f32x16{} : st[0][q & 1], 0, 0, 0);
           kb += TB;
           mask(st[0], 0);
-          m = row_max(st[0]) + (safe ? 0.f : P64Rows<E>::kMaxLift);
+          m = row_max(st[0]) + (safe ? 0.f : kMaxLift);
         }
         if constexpr (KG == 2) {
           if (!safe) {  // group 0's max for both (a wave without a tile there has none here)

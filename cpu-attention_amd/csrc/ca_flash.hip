@@ -78,18 +78,20 @@ __host__ __device__ inline BlockWork block_work(const FlashParams& p, int64_t bi
 // constant.  The V^T MFMA operands come from ds_read_b64_tr_b16 on the row-major
 // V tile: it gives lane j of a 16-lane group column j of a 4-row x 16-column
 // block (4 keys of one dim).
+constexpr int kTileKeys = 64;  // keys per bf16 tile, of both kernels
 template <int E>
 struct FlashBf16Cfg {
+  static_assert(E == 128, "duo_plan leaves no other head dim to the 64-row kernel");
   static constexpr int NWG = 4;            // waves that share a tile's loads
-  static constexpr int BN = 64;            // keys per tile
+  static constexpr int BN = kTileKeys;
   static constexpr int CPR = E / 8;        // 16-byte chunks per row
   // Padded row strides in chunks.  K: 16 lanes reading one 16-byte column of 16
   // consecutive rows hit 16 different 4-bank groups.  V: the 32 lanes that a
   // transposed read serves together read 4 rows x two 32-byte segments; a stride
-  // of 4 or 12 chunks mod 16 puts the 4 rows 16 banks apart, so the 8 segments
-  // cover the 64 banks once.
+  // of 4 chunks mod 16 puts the 4 rows 16 banks apart, so the 8 segments cover the
+  // 64 banks once.
   static constexpr int RSK = CPR + 1;
-  static constexpr int RSV = CPR == 16 ? 20 : (CPR == 8 ? 12 : 4);
+  static constexpr int RSV = CPR + 4;
   // Direct loads per thread and tile: the 4 waves load a tile, every load of a
   // wave fills 64 consecutive chunks, so a tile buffer is NL rounds of 4 x 64
   // chunks.  K and V tiles take the same NL (the larger), so every wave issues
@@ -227,7 +229,7 @@ __host__ __device__ inline void tile_offsets(int wv4, int lane, int stride, int 
 // the range is empty.
 template <int E>
 __host__ __device__ inline int tile_window(int rows, int stride2) {
-  return rows >= FlashBf16Cfg<E>::BN ? 0x7fffffff : (rows <= 0 ? 0 : (rows - 1) * stride2 + E * 2);
+  return rows >= kTileKeys ? 0x7fffffff : (rows <= 0 ? 0 : (rows - 1) * stride2 + E * 2);
 }
 
 // One wave's share of the successive K tiles or V tiles of a pass: rows [k0, k0 + BN) of the source per tile, cut at the pass's key
@@ -515,6 +517,10 @@ struct FlashP64Cfg {
   static_assert(LDS_BYTES + 1024 <= 160 * 1024, "tile buffers fit the LDS with room for the block's own");
 };
 
+// How far above its first tile's a fast walk fixes a row's max, in log2 units (see
+// P64Rows::fix_max; flash_duo_kernel's walks too).
+constexpr float kMaxLift = 64.f;
+
 // 64 query rows of one (batch, head) as two 32-row column blocks cb: lane (query
 // li, half hf) of block cb holds row r0 + 32 cb + li.
 template <int E>
@@ -662,7 +668,6 @@ struct P64Rows {
   // tile 0's max (64 without the lift); only rows whose logits outgrow that go
   // through the safe pass.  False: a row sees keys of tile 0, but no finite logit (the
   // max would be fixed at 0, and p of later logits far below 0 flush).
-  static constexpr float kMaxLift = 64.f;
   __device__ __forceinline__ bool fix_max(const Bf16Pass& a, int kbeg) {
     bool fine = true;
 #pragma unroll
@@ -1255,14 +1260,14 @@ template <int E>
 static int bf16_launch(const FlashParams& p, const FlashPlan& plan, hipStream_t stream) {
   const DuoPlan d = duo_plan(p, E, plan);
   const int64_t splits = d.kg ? d.splits : plan.splits;
-  constexpr int threads = 64 * FlashP64Cfg<E>::NW, lds = FlashP64Cfg<E>::LDS_BYTES;
-  int st;
-  if (d.kg)
+  int st = CA_DECLINED;  // E < 128 and more blocks than a grid takes (no memory holds such a call)
+  if (d.kg) {
     st = duo_launch<E>(p, d, stream);
-  else if (plan.split)
-    st = launch_lds(flash_bf16_p64_kernel<E, true>, plan.gx, threads, lds, p, stream, splits);
-  else
-    st = launch_lds(flash_bf16_p64_kernel<E, false>, plan.gx, threads, lds, p, stream);
+  } else if constexpr (E == 128) {
+    constexpr int threads = 64 * FlashP64Cfg<E>::NW, lds = FlashP64Cfg<E>::LDS_BYTES;
+    st = plan.split ? launch_lds(flash_bf16_p64_kernel<E, true>, plan.gx, threads, lds, p, stream, splits)
+                    : launch_lds(flash_bf16_p64_kernel<E, false>, plan.gx, threads, lds, p, stream);
+  }
   return st == CA_OK && splits > 1 ? flash_combine_launch(p, E, true, splits, stream) : st;
 }
 
