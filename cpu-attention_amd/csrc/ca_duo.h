@@ -421,23 +421,25 @@ __global__ __launch_bounds__(256 * KG, (DuoCfg<E, KG>::WAVES)) void flash_duo_ke
       int t = 0;
       if (nkt > 0) {
         loads_landed_barrier<2 * NL>();  // K(0) has landed
-        if (nkt_w > 0) {
+        auto first = [&]() __attribute__((always_inline)) {
 #pragma unroll
           for (int q = 0; q < NS2; ++q)
             st[0][q & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kread(kb, q), qr[q >> 1], q < 2 ? f32x16{} : st[0][q & 1], 0, 0, 0);
           kb += TB;
           mask(st[0], 0);
           m = row_max(st[0]) + (safe ? 0.f : kMaxLift);
-        }
-        if constexpr (KG == 2) {
+        };
+        if (KG == 2) {
+          if (nkt_w > 0) first();
           if (!safe) {  // group 0's max for both (a wave without a tile there has none here)
-            float* first = reinterpret_cast<float*>(duo_smem + C::TILES) + 32 * wv + li;
-            if (grp == 0) *first = m;
+            float* fixed = reinterpret_cast<float*>(duo_smem + C::TILES) + 32 * wv + li;
+            if (grp == 0) *fixed = m;
             __syncthreads();
-            m = *first;
+            m = *fixed;
           }
         }
         if (nkt_w > 0) {
+          if (KG == 1) first();
           nmu = m == -INFINITY ? 0.f : -m;
           // No finite logit among the first tile's visible keys: the max would be fixed
           // at 0, and p of later logits far below 0 flush.
