@@ -51,13 +51,13 @@
 // Key groups (KG = 2): a second set of 4 waves on the same rows walks every other tile
 // and merges in LDS, as in flash_duo_kernel, for grids that give a CU one block: the
 // waves of one block do not cover each other's softmax and splitting (N=1 L=S=2048 H=32
-// E=128 causal, 256 pairs: 171 -> 139 us; L=S=4096 H=16 E=64 196 -> 143 us).
+// E=128 causal, 256 pairs: 171 -> 139 us; L=S=4096 H=16 E=64 196 -> 146 us).
 //
 // Bound: the three MFMAs per product and the splitting of K and V tiles by every block
-// of 128 rows.  Measured back to back, before -> now: N=1 L=S=2048 H=32 E=128 causal 330
-// -> 139 us (246 TFLOP/s), N=1 L=S=4096 non-causal 2094 -> 947 us (290 TFLOP/s), N=4
-// L=S=4096 H=32 E=64 causal 2266 -> 1136 us, N=8 L=S=512 H=16 E=64 81 -> 43 us, N=1 L=64
-// S=4096 H=8 E=64 30 -> 21 us.
+// of 128 rows.  Measured back to back, 32-bit MFMAs -> now: N=1 L=S=2048 H=32 E=128
+// causal 330 -> 139 us (248 TFLOP/s), N=1 L=S=4096 non-causal 2077 -> 909 us (303
+// TFLOP/s), N=4 L=S=4096 H=32 E=64 causal 2244 -> 1099 us, N=8 L=S=512 H=16 E=64 81 -> 42
+// us, N=1 L=64 S=4096 H=8 E=64 29 -> 21 us.
 #pragma once
 
 namespace ca {

@@ -7,9 +7,10 @@
 //
 // bf16 calls take one of two tiled kernels (duo_plan in ca_duo.h): flash_duo_kernel
 // for most, and for long E = 128 walks that fill the chip flash_bf16_p64_kernel: 4
-// waves x 64 query rows per block, one wave per SIMD.  A wave's VALU work runs while its own independent MFMAs
-// execute, so each wave issues one stream per key tile of 64: the P.V MFMAs of
-// the previous tile, the S MFMAs of the next and the softmax of this one.  Key
+// waves x 64 query rows per block, one wave per SIMD.  A wave's VALU work runs while
+// its own independent MFMAs execute, so each wave issues one stream per key tile of
+// 64: the P.V MFMAs of the previous tile, the S MFMAs of the next and the softmax of
+// this one.  Key
 // tiles go global -> LDS with direct buffer loads; K is read with ds_read_b128,
 // V^T with ds_read_b64_tr_b16 from the row-major V tile.
 //   S^T = K Q^T   32x32x16 MFMAs with keys as rows and queries as columns, so a
@@ -21,8 +22,9 @@
 //   O^T += V^T P^T the probabilities are already in the B-operand layout of the
 //                 MFMA (no LDS round trip); P is rounded to bf16 as the reference's
 //                 bf16 policy does (flash_vec.mojo:255-259), fp32 accumulation.
-// fp32 (flash_f32_kernel): 4 waves x 32 rows, K/V staged through registers into
-// LDS, v_mfma_f32_32x32x2_f32, everything fp32.
+// fp32 (flash_f32_kernel, ca_f32.h): 4 or 8 waves x 32 rows, K/V staged through
+// registers into LDS, products from two fp16 halves per operand on the fp16 MFMAs with
+// fp32 sums; few keys, and values the halves do not serve, on v_mfma_f32_32x32x2_f32.
 #include <type_traits>
 
 #include "ca_device.h"
@@ -659,9 +661,9 @@ struct P64Rows {
   }
 
   // Fixes each row's max at kMaxLift above tile 0's (every row that sees any key of
-  // [kbeg, ..) sees key kbeg), in scaled log2 units as the reference takes it.  The softmax is
-  // the same for any max; the lift only moves the window of logits the fixed max
-  // serves exactly.  p of tile 0's largest logit is 2^-64, so p stays a normal
+  // [kbeg, ..) sees key kbeg), in scaled log2 units as the reference takes it.  The
+  // softmax is the same for any max; the lift only moves the window of logits the fixed
+  // max serves exactly.  p of tile 0's largest logit is 2^-64, so p stays a normal
   // fp32 (and bf16) for logits down to 62 below it: smaller ones weigh less than
   // 2^-62 against that key and may flush to 0.  Upwards, a lane's sum of p over a
   // tile stays within the walk's 2^64 headroom for logits up to about 123 above
