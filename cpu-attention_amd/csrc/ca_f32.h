@@ -15,7 +15,8 @@
 // rows) 1.6e-6 -> 6.9e-7, 2.0e-6 -> 9.3e-7, 1.0e-6 -> 5.0e-7; with lognormal V 4.8e-7 ->
 // 1.6e-7, 9.5e-7 -> 6.0e-7, 1.7e-7 -> 1.2e-7.  Over few keys the chains are short and
 // the splits would lose up to 45 % (E=64 L=S=17 causal 1.2e-7 -> 1.7e-7): f32_exact
-// leaves those calls to the 32-bit MFMAs.
+// leaves those calls to the 32-bit MFMAs (E=64 causal up to 56 keys: N=8 H=16 L=S=48 9.6
+// us there, 8.5 here; N=16 H=32 L=S=56 14.8, 11.3).
 //
 // Range.  fp16 reaches from 2^-24 to 65504, so the operands are scaled by powers of two:
 // each Q row by its own maximum, K and V by that of the range's first tile, to [2^10,
@@ -32,21 +33,23 @@
 //           largest |O| has to be 2^23.8 times the first (sum p'^2 <= 2^14 sum p') and
 //           2^22.8 times the second: kF32RowSum, kF32RowKeys.  So rows whose weight lies
 //           on keys of much smaller values, or of none, are redone.
-//   columns of V must not hide behind larger ones: in every whole tile, of the 8 keys that
-//           a wave stages, one reaches 2^-3 (kF32Dense) in each column, whose quanta then
-//           stay below 2^-21.3 of it.  Columns that are 0 in the first tile must be 0 in
-//           all (padded head dims), and 8 keys of zeros pass (padded keys).  A column of
-//           zeros in some tiles only (a one-hot V, say) is redone: where the others have
-//           none, it consists of P's small values, which are quanta themselves.
+//   columns of V must not hide behind larger ones: in every tile (of kF32TileKeys or more
+//           keys), of the 8 keys that a wave stages, one reaches 2^-3 (kF32Dense) in each
+//           column, whose quanta then stay below 2^-21.3 of it.  Columns that are 0 in the
+//           first tile must be 0 in all (padded head dims), and 8 keys of zeros pass
+//           (padded keys).  A column of zeros in some tiles only (a one-hot V, say) is
+//           redone: where the others have none, it consists of P's small values, which
+//           are quanta themselves.
 // (A single value far below both its row's and its column's others keeps its quantum's
 // error, small against theirs.)
-//   others: a K or V first tile of zeros or past the last key, a maximum outside 2^-40 ..
+//   others: a K or V first tile of zeros or of too few keys, a maximum outside 2^-40 ..
 //           2^40, a later tile's past 2^5 times the first's, inf or NaN.
 // What the first tile shows costs that tile alone (E=64 L=1024 S=8192 H=8, a V channel 1e4
 // times the others: 165 us, N(0, 1) 85, 32-bit MFMAs 156), the rest the walk.  Channels of
 // K 20 or of V 100 times the others, q 30 times larger or one value of 300 stay on the
 // split operands.  The checks cost 0 to 4 % (N=1 L=S=2048 H=32 E=128 causal 147.0 -> 147.8
-// us, N=8 L=S=512 H=16 E=64 35.7 -> 37.1, N=1 L=17 S=4096 H=8 E=128 27.6 -> 28.8).
+// us, N=8 L=S=512 H=16 E=64 35.7 -> 37.1, N=1 L=17 S=4096 H=8 E=128 27.6 -> 28.8; N=2
+// L=S=17 H=16 E=128 8.2 -> 8.6).
 //
 // Key groups (KG = 2): a second set of 4 waves on the same rows walks every other tile
 // and merges in LDS, as in flash_duo_kernel, for grids that give a CU one block: the
@@ -153,12 +156,21 @@ struct F32Cols {
   }
 };
 
-// Calls of few keys stay on the 32-bit MFMAs, which are closer to 64 bits there and no
-// slower (E=32 L=S=17: 4.5 against 5.4 us; E=32 L=S=200 causal error 1.9e-7 against
-// 2.0e-7, non-causal from 48 keys lower; E=64 L=S=32 causal 1.57e-7 against 1.68e-7,
-// from 40 keys even), and calls without a whole key tile have to.
+// Keys that a tile needs for a look at V's columns: 4 or more of them lie in every wave's
+// rows then, at E = 32 in whole tiles alone.
+template <int E>
+constexpr int kF32TileKeys = E == 32 ? 32 : 16;
+
+// Calls of few keys stay on the 32-bit MFMAs, which are closer to 64 bits there (N(0, 1),
+// L=S: E=32 causal 160 keys 1.85e-7 against 1.9e-7 and more, 193 even, non-causal 48 keys
+// 2.17e-7 against 2.20e-7, 64 2.35e-7 against 2.30e-7; E=64 causal 48 keys 1.69e-7 against
+// 1.72e-7, 64 1.81e-7 against 1.78e-7, non-causal from 33 keys 2.46e-7 against 2.15e-7)
+// and up to 32 keys no slower (E=32 L=S=17 4.5 against 5.4 us), as do calls of too few
+// keys for a tile.
 inline bool f32_exact(int E, bool causal, int64_t seq_k) {
-  return E == 32 ? seq_k <= (causal ? 192 : 32) : seq_k <= (E == 64 ? 32 : 31);
+  if (E == 32) return seq_k <= (causal ? 192 : 56);
+  if (E == 64) return seq_k <= (causal ? 56 : 32);
+  return seq_k < kF32TileKeys<128>;
 }
 
 template <int E, int KG, bool SPLIT>
@@ -220,9 +232,9 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
     };
     auto load_k = [&](int t, u32x4 (&x)[CH]) __attribute__((always_inline)) { load_one(kg, p.ks[1], koff, kstep, t, x); };
     auto load_v = [&](int t, u32x4 (&x)[CH]) __attribute__((always_inline)) { load_one(vg, p.vs[1], voff, vstep, t, x); };
-    // Not ok: the split operands do not serve the query block (Range, above).  A range
-    // whose first tile is not whole has no tile to judge V's columns by.
-    bool ok = nkt == 0 || kbeg + (grp + 1) * BN <= S;
+    // Not ok: the split operands do not serve the query block (Range, above).
+    auto judged = [&](int t) __attribute__((always_inline)) { return S - (kbeg + (t * KG + grp) * BN) >= kF32TileKeys<E>; };
+    bool ok = nkt == 0 || judged(0);
     float sk = 1.f, sv = 1.f;
     uint32_t* xw = reinterpret_cast<uint32_t*>(f32_smem + C::tiles(KG)) + grp * 4 * C::XW;
     bool zeros = false;  // some columns of the first V tile are all 0
@@ -280,7 +292,7 @@ __global__ __launch_bounds__(256 * KG, 2) void flash_f32_kernel(FlashParams p, i
       const uint32_t t0 = top.x, t1 = top.y;
       vsum = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, t0), __builtin_bit_cast(f16x2, t0), vsum, false);
       vsum = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, t1), __builtin_bit_cast(f16x2, t1), vsum, false);
-      if (kbeg + (t * KG + grp + 1) * BN > S) return;
+      if (!judged(t)) return;
       const uint32_t r[4] = {F32Cols<E>::of((top.x & 0xffff) >= kF32Dense), F32Cols<E>::of((top.x >> 16) >= kF32Dense),
                              F32Cols<E>::of((top.y & 0xffff) >= kF32Dense), F32Cols<E>::of((top.y >> 16) >= kF32Dense)};
       if (__builtin_expect((r[0] & r[1] & r[2] & r[3]) == F32Cols<E>::ALL && !zeros, 1)) return;

@@ -164,12 +164,12 @@ def test_values_of_very_different_size(cuda, d, what, shape, r):
 
 
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("shape", [(1, 40, 31, 3), (1, 40, 5, 3), (1, 17, 32, 2), (2, 33, 60, 3), (1, 40, 2049, 3),
-                                   (1, 300, 260, 30)])
+@pytest.mark.parametrize("shape", [(1, 40, 31, 3), (1, 40, 16, 3), (1, 40, 15, 3), (1, 40, 5, 3), (1, 17, 32, 2),
+                                   (2, 33, 60, 3), (1, 40, 2049, 3), (1, 40, 2064, 3), (1, 300, 260, 30)])
 @pytest.mark.parametrize("d", [32, 64, 128])
 def test_a_channel_in_few_keys(cuda, d, shape, causal):
-    """No whole key tile, one and a part of one, a split that holds a part alone, and
-    more rows than keys."""
+    """No whole key tile, one and a part of one, splits that hold a part alone (too few
+    keys to judge a channel by, and just enough), and more rows than keys."""
     q, k, v = tensors(shape, d, d + 6, cuda)
     v = _channel(v, 5, 1e-7)
     heads = some_heads(shape[3])
